@@ -382,7 +382,7 @@ int xrmm_gather_block_quantized(const void* data, const void* indices, int32_t i
 int xrmm_matmul_bnb4(const void* A, const void* B, const void* absmax, void* Y, int64_t M, int64_t K, int64_t N,
                      int32_t block_size, int32_t quant_type, int32_t trans_b, int32_t dtype, void* stream);
 
-/* Kernel family xrmm_matmul_bnb4 picks ("bnb4_gemv" or "bnb4_scalar"), NULL
+/* Kernel family xrmm_matmul_bnb4 picks ("bnb4_gemm", "bnb4_gemv" or "bnb4_scalar"), NULL
  * for an invalid geometry. No device work. */
 const char* xrmm_matmul_bnb4_kernel(int64_t M, int64_t K, int64_t N, int32_t block_size, int32_t quant_type,
                                     int32_t trans_b, int32_t dtype);

@@ -1,0 +1,105 @@
+"""GPU: the K-split block-scaled GEMM (MatMulBnb4 with float16 activations and
+five or more rows; int8-activation MatMulNBits with many rows) at the edges of
+its tiles: one and a few rows past a 32-row tile, columns past a wave's 32, K of
+one pair of 64-code steps, of a half step and of uneven groups, every block
+mode. MatMulBnb4 and the int8 path are compared with float64 at the bound of one
+binary16 rounding plus float32 sums over K; infinities reach the sums as the
+products do."""
+import numpy as np
+import pytest
+
+from oracle import int8a as Q8
+from oracle import oracle as O
+from oracle import quant as Q
+
+pytestmark = pytest.mark.gpu
+torch = pytest.importorskip("torch")
+
+
+def ops():
+    from xrgpu_amd import ops as _ops
+    return _ops
+
+
+def dev(a):
+    return None if a is None else torch.from_numpy(np.ascontiguousarray(a)).cuda()
+
+
+def close(got, exact, mag, K, half):
+    """One rounding of the result (2^-11 or 2^-24 of it), float32 sums and the
+    codebook terms' 2^-22: K + 4 units of 2^-24 of the sum of magnitudes at most."""
+    lim = np.abs(exact) * (2.0 ** -11 if half else 2.0 ** -24) + mag * ((K + 4) * 2.0 ** -24) + 2.0 ** -24
+    err = np.abs(got.astype(np.float64) - exact)
+    assert np.all(err <= lim), float((err - lim).max())
+
+
+BNB = [  # M, K, N, block, quant_type
+    (5, 32, 1, 32, 1),          # half a step
+    (5, 96, 33, 32, 0),         # K not a multiple of 64
+    (32, 128, 32, 64, 1),       # one pair of steps
+    (33, 192, 65, 64, 0),       # second row tile of one row; K not a multiple of 128
+    (64, 1024, 130, 128, 1),
+    (97, 1152, 257, 128, 1),    # 18 steps
+    (130, 2048, 100, 256, 0),
+    (250, 4096, 512, 64, 1),
+    (129, 1088, 2100, 32, 1),   # 17 steps over the groups
+    (3, 14336, 40, 64, 1),      # rows that do not fit the GEMV's LDS
+]
+
+
+@pytest.mark.parametrize("M,K,N,bs,qt", BNB)
+def test_bnb4(gpu, M, K, N, bs, qt):
+    rng = np.random.default_rng(M + K + N + bs)
+    a = rng.standard_normal((M, K)).astype(np.float16)
+    b = rng.integers(0, 256, N * K // 2, dtype=np.uint8)
+    s = rng.uniform(0.02, 1.5, N * K // bs).astype(np.float16)
+    assert ops().bnb4_kernel(M, K, N, bs, qt, 1, torch.float16) == "bnb4_gemm"
+    got = ops().matmul_bnb4(dev(a), dev(b), dev(s), K=K, N=N, block_size=bs, quant_type=qt).cpu().numpy()
+    codes = np.stack((b >> 4, b & 15), -1).reshape(N, K)
+    W = (Q.NF4 if qt == 1 else Q.FP4).astype(np.float64)[codes] * np.repeat(s.astype(np.float64).reshape(N, -1), bs, 1)
+    close(got, a.astype(np.float64) @ W.T, np.abs(a).astype(np.float64) @ np.abs(W).T, K, True)
+
+
+@pytest.mark.parametrize("qt", [1, 0])
+def test_bnb4_nonfinite(gpu, qt):
+    """An infinite or NaN activation gives what its products give: code by code."""
+    M, K, N, bs = 6, 128, 16, 32
+    a = np.ones((M, K), np.float16)
+    a[1, 3], a[2, 70], a[3, 127], a[4, 0] = np.inf, -np.inf, np.nan, 65504
+    b = np.zeros((N, K // 2), np.uint8)
+    b[:] = (np.arange(N, dtype=np.uint8) * 17)[:, None]  # column n holds code n everywhere
+    s = np.full(N * K // bs, 0.5, np.float16)
+    got = ops().matmul_bnb4(dev(a), dev(b.reshape(-1)), dev(s), K=K, N=N, block_size=bs, quant_type=qt).cpu().numpy()
+    ref = Q.matmul_bnb4(a, b.reshape(-1), s, K=K, N=N, block_size=bs, quant_type=qt)
+    assert np.array_equal(np.isnan(got), np.isnan(ref))
+    assert np.array_equal(got[np.isinf(ref)], ref[np.isinf(ref)])
+    fin = np.isfinite(ref)
+    assert np.allclose(got[fin].astype(np.float64), ref[fin].astype(np.float64), rtol=2e-3, atol=1e-3)
+
+
+I8A = [  # M, K, N, block, zero points, bias, dtype
+    (2049, 128, 1030, 32, True, True, np.float16),   # one pair of steps
+    (33, 1024, 8200, 64, True, False, np.float32),
+    (97, 1152, 2500, 128, True, True, np.float16),   # nine activation blocks over the groups
+    (65, 2176, 2001, 32, False, True, np.float32),
+    (8, 8192, 4100, 256, True, False, np.float16),
+]
+
+
+@pytest.mark.parametrize("M,K,N,bs,zp,bias,dt", I8A)
+def test_int8a(gpu, M, K, N, bs, zp, bias, dt):
+    assert M >= 8 and M * K * N >= 1 << 28  # the GEMM takes it
+    rng = np.random.default_rng(M + K + N + bs)
+    kb = K // bs
+    A = (rng.standard_normal((M, K)) * rng.uniform(0.2, 4, (M, 1))).astype(dt)
+    B = rng.integers(0, 256, (N, kb, bs // 2), dtype=np.uint8)
+    S = rng.uniform(0.005, 0.05, (N, kb)).astype(dt)
+    Z = rng.integers(0, 256, (N, (kb + 1) // 2), dtype=np.uint8) if zp else None
+    b = (rng.standard_normal(N) * 0.1).astype(dt) if bias else None
+    got = ops().matmul_nbits_int8a(dev(A), dev(B), dev(S), dev(Z), dev(b), K=K, N=N, block_size=bs).cpu().numpy()
+    kind = O.ZP_PACKED if zp else None
+    ref = Q8.matmul_nbits_int8a(A, B, S, Z, b, K=K, N=N, block_size=bs, zp_kind=kind, out_dtype=np.float64)
+    q, sa = Q8.quantize_activations(A, K)
+    W = O.dequantize(B, S, Z, K, 4, bs, kind).astype(np.float64)
+    mag = np.abs(q.astype(np.float64) * np.repeat(sa.astype(np.float64), 128, 1)) @ np.abs(W).T
+    close(got, ref, mag, K // 16, dt == np.float16)  # block sums are exact: a few roundings per block

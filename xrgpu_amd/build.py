@@ -51,6 +51,8 @@ UNITS = [
     ("xrmm_moe.hip", [], "moe.o"),
     ("xrmm_quant.hip", [], "quant.o"),
     ("xrmm_int8a.hip", [], "int8a.o"),
+    ("xrmm_bnb4_gemm.hip", [], "bnb4_gemm.o"),
+    ("xrmm_int8a_gemm.hip", [], "int8a_gemm.o"),
     ("xrmm_probe.hip", [], "probe.o"),
     ("xrmm_api.cpp", [], "api.o"),
     ("xrmm_operator.cpp", [], "operator.o"),

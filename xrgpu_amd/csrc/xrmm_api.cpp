@@ -604,7 +604,7 @@ const char* xrmm_matmul_bnb4_kernel(int64_t M, int64_t K, int64_t N, int32_t blo
   a.A = probe;
   a.B = probe;
   ok();
-  return xrmm::bnb4_fast_ok(a) ? "bnb4_gemv" : "bnb4_scalar";
+  return xrmm::bnb4_gemm_ok(a) ? "bnb4_gemm" : xrmm::bnb4_fast_ok(a) ? "bnb4_gemv" : "bnb4_scalar";
 }
 
 // ---------------------------------------------------------------------------

@@ -10,7 +10,8 @@
 //    32 codes, convert the column's codes once to signed bytes (code - zero:
 //    (c | 0x80) - z, then ^ 0x80, per byte without borrows), and for each row
 //    form exact int32 chunk sums with v_dot4_i32_i8, scaled by the weight
-//    block's and the activation block's scales in float32.
+//    block's and the activation block's scales in float32. Calls with many rows
+//    take the matrix cores instead (xrmm_int8a_gemm.hip).
 #include <atomic>
 #include <mutex>
 
@@ -109,6 +110,7 @@ hipError_t launch_t(const Int8aArgs& a, hipStream_t st) {
   const int64_t blocks = a.M * (a.K / kI8aBlock);
   hipLaunchKernelGGL(k_i8a_quant<T>, dim3(static_cast<uint32_t>((blocks + 3) / 4)), dim3(I8T), 0, st, a);
   if (hipError_t e = hipGetLastError(); e != hipSuccess) return e;
+  if (i8a_gemm_ok(a)) return launch_i8a_gemm(a, st);
   const dim3 grid(static_cast<uint32_t>((a.N + 3) / 4));
   const int64_t cpl = (a.K / 32 + 63) / 64;
   if (cpl <= 1) hipLaunchKernelGGL((k_i8a_gemv<T, 1>), grid, dim3(I8T), 0, st, a);

@@ -32,6 +32,15 @@ struct Bnb4Args {
   int bs, qt, tb, f16;
 };
 
+// Rows from which MatMulBnb4 with float16 activations takes the matrix cores: five,
+// where the GEMV would go over the weights a second time (K = N = 4096: 16.4 us
+// against 12.9; K = 4096, N = 14336: 35.7 against 21; K = N = 1024: 10.4 against 7.6),
+// or wherever its staged rows do not fit the LDS (K = 14336 from three rows on, left
+// to one thread per output otherwise).
+constexpr int64_t kBnb4GemmMinM = 5;
+bool bnb4_gemm_ok(const Bnb4Args& a);
+hipError_t launch_bnb4_gemm(const Bnb4Args& a, const float (&nf4)[16], const float (&fp4)[16], hipStream_t st);
+
 bool bnb4_fast_ok(const Bnb4Args& a);
 hipError_t launch_bnb4(const Bnb4Args& a, hipStream_t st);
 
@@ -62,6 +71,15 @@ struct Int8aArgs {
 inline int64_t i8a_workspace_bytes(int64_t M, int64_t K) {
   return (M * K + 255) / 256 * 256 + M * (K / kI8aBlock) * 4;
 }
+
+// Multiply-adds (and rows) from which the int8-activation path takes the matrix
+// cores: the GEMV's time grows with rows x weights, the GEMM's hardly below 32 rows.
+// K = N = 4096: 12.1 us (8 rows), 14.5 (16), 19.2 (24) against 13.7, 14.2, 14.7;
+// K = 4096, N = 14336: 23.4 (8), 39.4 (16) against 20.5, 21; K = 14336, N = 1024:
+// 24 (8), 43 (16) against 34, 35.
+constexpr int64_t kI8aGemmMinMacs = int64_t(1) << 28, kI8aGemmMinM = 8;
+bool i8a_gemm_ok(const Int8aArgs& a);
+hipError_t launch_i8a_gemm(const Int8aArgs& a, hipStream_t st);
 
 hipError_t launch_i8a(const Int8aArgs& a, hipStream_t st);
 

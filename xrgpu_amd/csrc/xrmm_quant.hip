@@ -19,8 +19,9 @@
 // codes with one 16-byte chunk (32 codes) per lane, looks codes up in a
 // 16-entry float32 table in LDS (exact reference values) and accumulates in
 // float32 against A rows staged in LDS; the absmax of a chunk multiplies the
-// chunk's partial sum. Everything else runs one thread per output element in
-// the reference's serial order.
+// chunk's partial sum. Five and more rows of float16 activations go to the matrix
+// cores (xrmm_bnb4_gemm.hip). Everything else runs one thread per output element
+// in the reference's serial order.
 #include "xrmm_device.h"
 #include "xrmm_quant.h"
 
@@ -31,12 +32,12 @@ namespace {
 constexpr int QT = 256;  // threads per workgroup
 
 // bitsandbytes codebooks (complex_kernel.glsl:82): NF4 (quant_type 1), FP4 (0)
-__constant__ float kNF4[16] = {-1.0f, -0.6961928009986877f, -0.5250730514526367f, -0.3949174880981445f,
+constexpr float kNF4[16] = {-1.0f, -0.6961928009986877f, -0.5250730514526367f, -0.3949174880981445f,
                                -0.28444138169288635f, -0.18477343022823334f, -0.09105003625154495f, 0.0f,
                                0.07958029955625534f, 0.16093020141124725f, 0.24611230194568634f,
                                0.33791524171829224f, 0.44070982933044434f, 0.5626170039176941f,
                                0.7229568362236023f, 1.0f};
-__constant__ float kFP4[16] = {0.0f, 0.0052083333333333f, 0.6666666666666666f, 1.0f, 0.3333333333333333f, 0.5f,
+constexpr float kFP4[16] = {0.0f, 0.0052083333333333f, 0.6666666666666666f, 1.0f, 0.3333333333333333f, 0.5f,
                                0.1666666666666666f, 0.25f, -0.0f, -0.0052083333333333f, -0.6666666666666666f,
                                -1.0f, -0.3333333333333333f, -0.5f, -0.1666666666666666f, -0.25f};
 
@@ -380,6 +381,7 @@ bool bnb4_fast_ok(const Bnb4Args& a) {
 
 hipError_t launch_bnb4(const Bnb4Args& a, hipStream_t st) {
   if (a.M == 0 || a.N == 0) return hipSuccess;
+  if (bnb4_gemm_ok(a)) return launch_bnb4_gemm(a, kNF4, kFP4, st);
   if (bnb4_fast_ok(a)) {
     const int mr = bnb4_rows_per_pass(a.M);
     if (a.f16) {
