@@ -1,0 +1,84 @@
+"""GPU: Qkv / Mlp on the 128-row tiles (normalised rows in a workspace, too few
+256 x 256 tiles for the large pipeline) against the oracle at the edges: a last
+row tile of one row, columns past a tile, K of one step, of an odd number of
+steps (uneven K groups) and with a last block that is not whole, narrow and wide
+tiles, every zero-point kind. Binary16 bar: max|d| <= 1e-2 max|Y|."""
+import numpy as np
+import pytest
+
+from oracle import oracle as O
+
+pytestmark = pytest.mark.gpu
+torch = pytest.importorskip("torch")
+
+
+def ops():
+    from xrgpu_amd import ops as _ops
+    return _ops
+
+
+def dev(a):
+    return None if a is None else torch.from_numpy(np.ascontiguousarray(a)).cuda()
+
+
+def weights(rng, N, K, bs, zp):
+    kb = (K + bs - 1) // bs
+    B = rng.integers(0, 256, (N, kb, bs // 2), dtype=np.uint8)
+    S = rng.uniform(0.001, 0.02, (N, kb)).astype(np.float16)
+    Z = None
+    if zp == "packed":
+        Z = rng.integers(0, 256, (N, (kb + 1) // 2), dtype=np.uint8)
+    elif zp == "float":
+        Z = rng.uniform(4, 12, (N, kb)).astype(np.float16)
+    return B, S, Z
+
+
+CASES = [  # M, K, N, Nkv, block, zero points, skip
+    (65, 64, 40, 8, 32, None, True),        # one step: the second K group has none
+    (129, 192, 130, 64, 32, "packed", False),  # three steps, a row tile of one row
+    (100, 1000, 257, 65, 64, "float", True),   # a last block that is not whole
+    (128, 2048, 512, 128, 128, None, False),
+    (385, 320, 9000, 136, 64, "packed", True),  # past one round of narrow tiles: wide ones
+    (257, 96, 11500, 64, 32, "float", False),
+]
+
+
+
+@pytest.mark.parametrize("M,K,N,Nkv,bs,zp,skip", CASES)
+def test_qkv(gpu, M, K, N, Nkv, bs, zp, skip):
+    rng = np.random.default_rng(M + K + N)
+    A = rng.standard_normal((M, K)).astype(np.float16)
+    sk = rng.standard_normal((M, K)).astype(np.float16) if skip else None
+    g = rng.uniform(0.5, 1.5, K).astype(np.float16)
+    q, k, v = (weights(rng, n, K, bs, zp) for n in (N, Nkv, Nkv))
+    kw = dict(q_zero_points=q[2], k_zero_points=k[2], v_zero_points=v[2])
+    got = ops().matmul_nbits_qkv(dev(A), dev(q[0]), dev(q[1]), dev(k[0]), dev(k[1]), dev(v[0]), dev(v[1]),
+                                 norm_scale=dev(g), skip=dev(sk), block_size=bs, **{n: dev(z) for n, z in kw.items()})
+    x = A.astype(np.float64) + (sk.astype(np.float64) if skip else 0)
+    x = (x / np.sqrt((x * x).mean(1, keepdims=True) + 1e-6) * g.astype(np.float64)).astype(np.float16)
+    for y, w, n in zip(got[:3], (q, k, v), (N, Nkv, Nkv)):
+        ref = O.matmul_nbits(x, w[0], w[1], w[2], None, K=K, N=n, block_size=bs)
+        ok, err, lim = O.tolerance_ok(y.cpu().numpy(), ref, np.float16)
+        assert ok, (err, lim)
+    r = (A.astype(np.float32) + (sk.astype(np.float32) if skip else np.float32(0))).astype(np.float16)
+    assert np.array_equal(got[3].cpu().numpy(), r)
+
+
+@pytest.mark.parametrize("M,K,N,Nkv,bs,zp,skip", CASES)
+def test_mlp(gpu, M, K, N, Nkv, bs, zp, skip):
+    rng = np.random.default_rng(M + K + N + 1)
+    A = rng.standard_normal((M, K)).astype(np.float16)
+    sk = rng.standard_normal((M, K)).astype(np.float16) if skip else None
+    g = rng.uniform(0.5, 1.5, K).astype(np.float16)
+    gw, uw = weights(rng, N, K, bs, zp), weights(rng, N, K, bs, zp)
+    gb, ub = ((rng.standard_normal(N) * 0.1).astype(np.float16) for _ in range(2))
+    y, _ = ops().matmul_nbits_mlp(dev(A), dev(gw[0]), dev(gw[1]), dev(uw[0]), dev(uw[1]), skip=dev(sk),
+                                  norm_scale=dev(g), gate_bias=dev(gb), up_bias=dev(ub), block_size=bs,
+                                  gate_zero_points=dev(gw[2]), up_zero_points=dev(uw[2]))
+    x = A.astype(np.float64) + (sk.astype(np.float64) if skip else 0)
+    x = (x / np.sqrt((x * x).mean(1, keepdims=True) + 1e-5) * g.astype(np.float64)).astype(np.float16)
+    h = [O.matmul_nbits(x, w[0], w[1], w[2], None, K=K, N=N, block_size=bs, out_dtype=np.float64) + b.astype(np.float64)
+         for w, b in ((gw, gb), (uw, ub))]
+    ref = h[0] / (1 + np.exp(-h[0])) * h[1]
+    ok, err, lim = O.tolerance_ok(y.cpu().numpy(), ref.astype(np.float16), np.float16)
+    assert ok, (err, lim)

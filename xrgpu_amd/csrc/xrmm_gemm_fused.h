@@ -1,4 +1,5 @@
-// MatMulNBitsQkv / MatMulNBitsMlp for more than 16 rows (prefill): a 128 x 128
+// MatMulNBitsQkv / MatMulNBitsMlp for more than 16 rows (prefill) without a
+// workspace for the normalised rows, or with blocks of 16: a 128 x 128
 // LDS-tiled GEMM with the operators' prologue and epilogue fused (fp16
 // activations, 4-bit weights, v_mfma_f32_32x32x16_f16, float32 accumulation).
 //

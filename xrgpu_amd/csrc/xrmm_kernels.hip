@@ -41,6 +41,7 @@
 #include "xrmm_gemv_sk.h"
 #include "xrmm_gemm.h"
 #include "xrmm_gemm_fused.h"
+#include "xrmm_gemm_mid.h"
 #include "xrmm_gemm_thin.h"
 
 namespace xrmm {
@@ -842,6 +843,11 @@ hipError_t launch(const Launch& L, hipStream_t st) {
       if (zpk == ZP_NONE) return launch_gemm_big_fused_for<ZP_NONE>(Lx, st);
       if (zpk == ZP_FLOAT) return launch_gemm_big_fused_for<ZP_FLOAT>(Lx, st);
       return launch_gemm_big_fused_for<ZP_PACKED>(Lx, st);
+    }
+    if (gemm_mid_ok(Lx)) {
+      if (zpk == ZP_NONE) return launch_gemm_mid_for<ZP_NONE>(Lx, st);
+      if (zpk == ZP_FLOAT) return launch_gemm_mid_for<ZP_FLOAT>(Lx, st);
+      return launch_gemm_mid_for<ZP_PACKED>(Lx, st);
     }
     if (zpk == ZP_NONE) return launch_gemm_fused_for<ZP_NONE>(Lx, st);
     if (zpk == ZP_FLOAT) return launch_gemm_fused_for<ZP_FLOAT>(Lx, st);
