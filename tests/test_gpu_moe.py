@@ -201,6 +201,31 @@ GROUPED_BLOCKS = [
 ]
 
 
+EDGES = [  # T, H, I, E, k, act, bits, bs: what the 128-pair tiles and super-steps of 256 codes cut
+    (32, 64, 64, 2, 1, "swiglu", 4, 0),       # one K step
+    (33, 320, 192, 1, 1, "swiglu", 4, 64),    # 33 pairs of one expert: two MFMA row tiles; five steps
+    (129, 576, 448, 1, 1, "relu", 4, 32),     # a second row tile of one pair; nine and seven steps
+    (97, 1344, 832, 3, 2, "swiglu", 4, 64),   # super-steps cut by the row's end, several to rotate over
+    (70, 1024, 1536, 4, 2, "relu", 4, 512),   # blocks longer than a super-step
+    (130, 704, 1216, 2, 2, "swiglu", 8, 64),
+    (64, 2560, 640, 5, 2, "swiglu", 8, 128),
+    (40, 8256, 128, 2, 2, "relu", 4, 0),      # rows read twice by the prologue
+]
+
+
+@pytest.mark.parametrize("T,H,I,E,k,act,bits,bs", EDGES)
+def test_grouped_edges(gpu, T, H, I, E, k, act, bits, bs):
+    """Float32 bar against the oracle at the edges of the grouped path's tiles."""
+    rng = np.random.default_rng(T * 3 + H + I + E + k + bits + bs)
+    sw = act == "swiglu"
+    i = rand_case(rng, T, H, I, E, bits, bs, sw)
+    at = dict(k=k, activation=act, swiglu_fusion=1 if sw else 0, bits=bits, block_size=bs, alpha=1.702 if sw else 1.0,
+              beta=1.0 if sw else 0.0, swiglu_limit=None)
+    assert ops().qmoe_kernel(T, H, E, 2 * I if sw else I, k, bits, bs, act, 1 if sw else 0) == "qmoe_grouped"
+    ok, err, lim = O.tolerance_ok(run_gpu(i, at), run_oracle(i, at), np.float32)
+    assert ok, f"max|d|={err} > {lim}"
+
+
 @pytest.mark.parametrize("T,H,I,E,k,act,bits,bs", GROUPED_BLOCKS)
 def test_grouped_block_scales(gpu, T, H, I, E, k, act, bits, bs):
     """Float32 bar against the oracle with per-block scales (each block's sum

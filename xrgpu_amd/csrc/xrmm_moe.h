@@ -56,11 +56,10 @@ constexpr int64_t kMoeGroupMaxExperts = 4096;
 // row exponents of x (T).
 inline int64_t moe_list_words(int64_t T, int64_t k) { return 2 * (kMoeGroupMaxExperts + 1) + 2 * T * k + T; }
 
-// K splits of the grouped path's FC2 GEMM (64-pair x 256-column tiles over
-// K = I): enough for about 512 workgroups (two per CU) when the pairs would
+// K splits of the grouped path's FC2 GEMM (64 pairs x 256 columns over K = I
+// as the unit): enough for about 512 workgroups (two per CU) when the pairs would
 // make fewer, four at most, each split at least 16 steps of 64. From the
-// geometry alone (one tile per 64 pairs), so the workspace bound and the
-// launch agree.
+// geometry alone, so the workspace bound and the launch agree.
 inline int64_t moe_group_fc2_splits(int64_t T, int64_t k, int64_t H, int64_t I) {
   const int64_t tiles = ((T * k + 63) / 64) * ((H + 255) / 256);
   if (tiles <= 0) return 1;

@@ -26,6 +26,7 @@
 // multiplies the sum of its block (or the row's total for row scales). Other
 // geometries take a routing kernel and one-thread-per-output kernels.
 #include <algorithm>
+#include <type_traits>
 
 #include "xrmm_device.h"
 #include "xrmm_moe.h"
@@ -39,10 +40,9 @@ constexpr int MOE_T = 256;  // threads per workgroup: 4 waves
 // ---------------------------------------------------------------------------
 // routing
 
-__global__ __launch_bounds__(MOE_T) void k_moe_route(const float* __restrict__ router, int32_t* __restrict__ sel,
-                                                     float* __restrict__ wts, int T, int E, int k) {
-  const int t = blockIdx.x * (MOE_T / 64) + (threadIdx.x >> 6), lane = threadIdx.x & 63;
-  if (t >= T) return;  // whole waves
+// One wave routes token t.
+__device__ void route_token(const float* __restrict__ router, int32_t* __restrict__ sel, float* __restrict__ wts, int t,
+                            int E, int k, int lane) {
   const float* l = router + static_cast<int64_t>(t) * E;
   auto rank_of = [&](int e, float v) {
     int r = 0;
@@ -93,6 +93,13 @@ __global__ __launch_bounds__(MOE_T) void k_moe_route(const float* __restrict__ r
   }
 }
 
+__global__ __launch_bounds__(MOE_T) void k_moe_route(const float* __restrict__ router, int32_t* __restrict__ sel,
+                                                     float* __restrict__ wts, int T, int E, int k) {
+  const int t = blockIdx.x * (MOE_T / 64) + (threadIdx.x >> 6), lane = threadIdx.x & 63;
+  if (t >= T) return;  // whole waves
+  route_token(router, sel, wts, t, E, k, lane);
+}
+
 // ---------------------------------------------------------------------------
 // row-group GEMV over packed expert rows
 
@@ -108,7 +115,7 @@ __device__ __forceinline__ float swiglu(float gate, float lin, const MoeArgs& a)
     lin = fminf(fmaxf(lin, -a.limit), a.limit);
   }
   const float z = a.alpha * gate;
-  const float lg = z >= 0.f ? 1.f / (1.f + expf(-z)) : expf(z) / (1.f + expf(z));
+  const float t = expf(-fabsf(z)), lg = (z >= 0.f ? 1.f : t) / (1.f + t);
   return gate * lg * (lin + a.beta);
 }
 
@@ -636,7 +643,7 @@ namespace {
 template <int ST, int BITS, int BKM>
 hipError_t mg_launch(const MoeArgs& a, const MgLists& g, int nct, int64_t grid, hipStream_t st) {
   auto kern = k_moe_ggemm<ST, BITS, BKM>;
-  constexpr size_t lds = mg_lds<BITS>();
+  constexpr size_t lds = mg_lds<BITS, BKM>();
   if constexpr (lds > 64 * 1024) {
     static std::atomic<int> done[kMaxDevices];  // per instantiation and device
     if (hipError_t e = raise_lds_cap(reinterpret_cast<const void*>(kern), static_cast<int>(lds), done); e != hipSuccess)
@@ -672,9 +679,11 @@ hipError_t launch_grouped(const MoeArgs& a0, hipStream_t st) {
   g.hmax = reinterpret_cast<uint32_t*>(g.list + a.T * a.k);
   g.ex = reinterpret_cast<int32_t*>(g.hmax + a.T * a.k);
   const int T = static_cast<int>(a.T), npairs = static_cast<int>(a.T * a.k), E = static_cast<int>(a.E);
-  hipLaunchKernelGGL(k_moe_route, dim3(static_cast<uint32_t>((a.T + 3) / 4)), dim3(MOE_T), 0, st, a.router, a.sel, a.wts,
-                     T, E, a.k);
-  hipLaunchKernelGGL(k_moe_xexp, dim3(static_cast<uint32_t>((a.T + 3) / 4)), dim3(256), 0, st, a.x, T, a.H, g.ex);
+  // x's terms go to yp (T k ks H floats), which FC2 overwrites
+  f16* xs = reinterpret_cast<f16*>(a.yp);
+  const int H = static_cast<int>(a.H);
+  auto prep = H <= 2048 ? k_moe_prep<1> : H <= 4096 ? k_moe_prep<2> : H <= 8192 ? k_moe_prep<4> : k_moe_prep<0>;
+  hipLaunchKernelGGL(prep, dim3(static_cast<uint32_t>(T)), dim3(256), 0, st, a.router, a.x, a.sel, a.wts, E, a.k, H, g.ex, xs);
   hipLaunchKernelGGL(k_moe_group, dim3(1), dim3(MG_T), 0, st, a.sel, npairs, E, g);
   if (hipError_t e = hipGetLastError(); e != hipSuccess) return e;
   // row tiles: at most one partial tile per expert beyond the full ones
@@ -684,8 +693,13 @@ hipError_t launch_grouped(const MoeArgs& a0, hipStream_t st) {
   const hipError_t e1 = a.act == XRMM_ACT_SWIGLU_CODE ? mg_launch_s<MG_FC1_SWIGLU>(a, g, nct1, rtmax * nct1, st)
                                                       : mg_launch_s<MG_FC1_RELU>(a, g, nct1, rtmax * nct1, st);
   if (e1 != hipSuccess) return e1;
+  const int64_t hg = a.T * a.k * (a.I / 8);
+  if ((hg + 255) / 256 > 0x7FFFFFFF) return hipErrorInvalidValue;
+  hipLaunchKernelGGL(k_moe_hsplit, dim3(static_cast<uint32_t>((hg + 255) / 256)), dim3(256), 0, st, a.h, g.hmax, hg,
+                     static_cast<int>(a.I / 8));
+  if (hipError_t e = hipGetLastError(); e != hipSuccess) return e;
   if (hipError_t e = mg_launch_s<MG_FC2>(a, g, nct2, rtmax * nct2 * a.ks, st); e != hipSuccess) return e;
-  hipLaunchKernelGGL(k_moe_combine, dim3(static_cast<uint32_t>((a.T * a.H + 255) / 256)), dim3(256), 0, st, a);
+  hipLaunchKernelGGL(k_moe_combine, dim3(static_cast<uint32_t>((a.T * (a.H / 4) + 255) / 256)), dim3(256), 0, st, a);
   return hipGetLastError();
 }
 }  // namespace

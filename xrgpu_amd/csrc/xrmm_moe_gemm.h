@@ -1,10 +1,11 @@
 // Grouped-expert QMoE for many tokens (included by xrmm_moe.hip): instead of
 // one pass over an expert's rows per (token, slot) pair, the pairs routed to
 // each expert are gathered into the rows of one GEMM per expert, so every
-// expert matrix is read once per 64 pairs.
+// expert matrix is read once per 128 pairs.
 //
-// Launches (row scales, 4-bit codes):
-//  1. routing (k_moe_route with the row exponents of x, below);
+// Launches:
+//  1. k_moe_prep: per token the routing, the row exponent of x, and x split into
+//     its binary16 terms (into yp, which nothing uses before FC2);
 //  2. k_moe_group: per-expert pair counts, offsets, row-tile offsets and the
 //     pair lists (one workgroup; the order of pairs inside a list does not
 //     change any result, every GEMM row being independent);
@@ -12,10 +13,11 @@
 //     its FC1 rows, K = H; the epilogue applies the row scale, the activation
 //     (SwiGLU rows 2j / 2j + 1 sit in neighbouring lanes) and writes h[pair],
 //     folding each pair's largest |h| into an arrival-order-free atomic max;
-//  4. k_moe_ggemm FC2: rows = the pairs' h, columns = the expert's FC2 rows,
+//  4. k_moe_hsplit: h into its binary16 terms, in place;
+//  5. k_moe_ggemm FC2: rows = the pairs' h, columns = the expert's FC2 rows,
 //     K = I, split over a.ks workgroups when the tiles are few; writes each
 //     split's yp[pair][split] (row scale applied);
-//  5. k_moe_combine: y[t] = sum over slots (ascending expert index) of
+//  6. k_moe_combine: y[t] = sum over slots (ascending expert index) of
 //     w * (the slot's splits summed in split order), one fused multiply-add
 //     per slot in slot order.
 //
@@ -27,27 +29,52 @@
 // MFMA takes hi and lo against the same weights, so each product keeps about
 // 22 bits of the activation, and the power of two is undone on the sum.
 // Non-finite activations keep lo = 0, so +-Inf and NaN reach the sums as the
-// reference's float32 products would.
+// reference's float32 products would. The terms take the place of the float32
+// values: the 256 bytes of 64 values hold their 64 hi, then their 64 lo, eight by
+// eight in the pair order of the dequantised codes, so the tiles stage them as they are
+// (split in the tiles, every column tile of an expert split the same rows again:
+// 40 of 180 VALU instructions a step).
+//
+// Tiles. 128 pairs x 256 columns, 8 waves of 2 x 4: a wave owns every other
+// 32-pair MFMA tile (two at most) and 64 columns, so a dequantised weight fragment
+// feeds two MFMA row tiles and experts with 1 .. 128 pairs cost ceil(pairs / 32)
+// MFMA tiles (the 64-pair tiles with two row groups of waves it replaces dequantised
+// every fragment twice and computed their empty rows). Mixtral's experts (H =
+// 4096, I = 14336, 8 experts, 2 taken, blocks of 64), 300 tokens:
+// 1.07 -> 0.74 ms (FC1 750 -> 500 us at best, FC2 338 -> 227, x's exponents by one wave a
+// token 28 us -> part of k_moe_prep's 8.5, combine 12.7 -> 6.5); 16 tokens 630 -> 376 us,
+// 2048 tokens 4.9 -> 3.5 ms. A step's time by wave: 1.7 - 2.0 k cycles of MFMAs and
+// dequantisation, 0.4 k issuing loads, 0.3 k staging, the rest barrier: the two waves of
+// a SIMD overlap only in part. One workgroup per CU leaves a tail where the tiles just
+// pass a round: row scales, ReLU, 250 pairs an expert and 4096 rows (1000 x 2048 x 4096,
+// 8 experts, 2 taken) take 286 us against 255 with 64-pair tiles, two workgroups per CU.
 #pragma once
 
 namespace xrmm {
 namespace {
 
-constexpr int MG_RT = 64;   // pairs per row tile
+constexpr int MG_RT = 128;  // pairs per row tile
 constexpr int MG_CT = 256;  // columns per tile
 constexpr int MG_K = 64;    // K step
 constexpr int MG_LD = MG_K + 8;
-constexpr int MG_T = 512;   // threads: 8 waves, 2 (rows of 32) x 4 (columns of 64)
-// halfs per stage: A hi, A lo (rows of MG_LD), then the raw codes as
-// [fragment of the step][column], a fragment being eight codes (one dword
-// of 4-bit codes, two of 8-bit codes)
+constexpr int MG_T = 512;   // threads: 8 waves, 2 (row tiles) x 4 (columns of 64)
+// Weights are staged for several K steps at once, a super-step: 128 bytes of every
+// column (256 codes of 4 bits, 128 of 8).
 template <int BITS>
-constexpr int mg_stage() {
-  return 2 * MG_RT * MG_LD + (MG_K / 8) * MG_CT * (BITS / 4) * 2;
+constexpr int mg_ss() {
+  return BITS == 4 ? 4 : 2;
 }
-template <int BITS>
+constexpr int MG_ASTAGE = 2 * MG_RT * MG_LD;  // halfs per A stage: hi, then lo (rows of MG_LD)
+constexpr int MG_WSTAGE = MG_CT * 128;        // bytes of a super-step's codes
+// scales of a column and super-step (block mode BKM: 2, 4, 8 = blocks of 32, 64, 128
+// or more codes; longer blocks repeat one scale)
+template <int BITS, int BKM>
+constexpr int mg_sb() {
+  return BKM == 0 ? 0 : BKM == 2 ? 2 * mg_ss<BITS>() : BKM == 4 ? mg_ss<BITS>() : mg_ss<BITS>() / 2;
+}
+template <int BITS, int BKM>
 constexpr size_t mg_lds() {
-  return 2 * mg_stage<BITS>() * sizeof(_Float16);
+  return 2 * (MG_ASTAGE * sizeof(_Float16) + MG_WSTAGE + mg_sb<BITS, BKM>() * MG_CT * sizeof(float));
 }
 
 // Block-scale modes of the GEMM: 0 = one scale per row (applied to the row's
@@ -74,19 +101,104 @@ __device__ __forceinline__ int mg_row_exp(float mx) {
   return e - 15;
 }
 
-// Row exponents of x: one wave per token, over the row's finite |x|.
-__global__ __launch_bounds__(256) void k_moe_xexp(const float* __restrict__ x, int T, int64_t H, int32_t* __restrict__ ex) {
-  const int t = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
-  if (t >= T) return;  // whole waves
-  const float* xr = x + static_cast<int64_t>(t) * H;
+// Eight values times 2^-e as their binary16 terms, hi then lo, in the codes' pair
+// order (0 4 1 5 2 6 3 7).
+__device__ __forceinline__ void mg_terms(const float (&x)[8], float scale, f16x8& hi, f16x8& lo) {
+#pragma unroll
+  for (int q = 0; q < 8; ++q) {
+    const float v = x[(q >> 1) + 4 * (q & 1)] * scale;
+    const f16 h = static_cast<f16>(v);
+    hi[q] = h;
+    lo[q] = __builtin_isfinite(v) ? static_cast<f16>(v - static_cast<float>(h)) : static_cast<f16>(0.f);
+  }
+}
+
+__device__ __forceinline__ void mg_load8(const float* p, float (&x)[8]) {
+  const f32x4 a = *reinterpret_cast<const f32x4*>(p), b = *reinterpret_cast<const f32x4*>(p + 4);
+  x[0] = a.x, x[1] = a.y, x[2] = a.z, x[3] = a.w, x[4] = b.x, x[5] = b.y, x[6] = b.z, x[7] = b.w;
+}
+
+// One workgroup per token: wave 0 routes it (k_moe_route's rule), every wave then
+// finds the row's largest finite |x|, and the row's terms go to xs [T][H] (256
+// bytes per 64 values). H % 64 == 0. P > 0: eight-value groups per thread in
+// registers (H <= 2048 P), the row read once; P == 0: any H, read twice.
+template <int P>
+__global__ __launch_bounds__(256) void k_moe_prep(const float* __restrict__ router, const float* __restrict__ x,
+                                                  int32_t* __restrict__ sel, float* __restrict__ wts, int E, int k,
+                                                  int H, int32_t* __restrict__ ex, f16* __restrict__ xs) {
+  __shared__ float red[4];
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int64_t t = blockIdx.x;
+  const float* row = x + t * H;
+  const int ng = H / 8;
+  float v[P > 0 ? P : 1][8];
   float m = 0.f;
-  for (int64_t i = lane; i < H; i += 64) {
-    const float v = __builtin_fabsf(xr[i]);
-    if (__builtin_isfinite(v)) m = fmaxf(m, v);
+  auto see = [&](const float (&a)[8]) {
+#pragma unroll
+    for (int q = 0; q < 8; ++q) {
+      const float u = __builtin_fabsf(a[q]);
+      if (__builtin_isfinite(u)) m = fmaxf(m, u);
+    }
+  };
+  if constexpr (P > 0) {
+#pragma unroll
+    for (int i = 0; i < P; ++i)
+      if (tid + 256 * i < ng) mg_load8(row + (tid + 256 * i) * 8, v[i]);
+#pragma unroll
+    for (int i = 0; i < P; ++i)
+      if (tid + 256 * i < ng) see(v[i]);
+  } else {
+    for (int g = tid; g < ng; g += 256) {
+      mg_load8(row + g * 8, v[0]);
+      see(v[0]);
+    }
   }
 #pragma unroll
   for (int off = 32; off > 0; off >>= 1) m = fmaxf(m, __shfl_xor(m, off, 64));
-  if (lane == 0) ex[t] = mg_row_exp(m);
+  if (lane == 0) red[tid >> 6] = m;
+  __syncthreads();
+  const int e = mg_row_exp(fmaxf(fmaxf(red[0], red[1]), fmaxf(red[2], red[3])));
+  const float scale = __builtin_ldexpf(1.f, -e);
+  if (tid == 0) ex[t] = e;
+  f16x8* out = reinterpret_cast<f16x8*>(xs + t * H * 2);
+  if constexpr (P > 0) {
+#pragma unroll
+    for (int i = 0; i < P; ++i)
+      if (tid + 256 * i < ng) {
+        f16x8 hi, lo;
+        mg_terms(v[i], scale, hi, lo);
+        const int g = tid + 256 * i, o = (g >> 3) * 16 + (g & 7);
+        out[o] = hi;
+        out[o + 8] = lo;
+      }
+  } else {
+    for (int g = tid; g < ng; g += 256) {
+      f16x8 hi, lo;
+      mg_load8(row + g * 8, v[0]);
+      mg_terms(v[0], scale, hi, lo);
+      out[(g >> 3) * 16 + (g & 7)] = hi;
+      out[(g >> 3) * 16 + (g & 7) + 8] = lo;
+    }
+  }
+  if (tid < 64) route_token(router, sel, wts, static_cast<int>(t), E, k, lane);
+}
+
+// h [T k][I] into its terms in place, eight values per thread; the row exponent from
+// the pair's largest |h| (FC1's atomic maximum). The eight threads that exchange
+// places inside 256 bytes are lanes of one wave (I % 64 == 0), whose load
+// instructions have all returned before its first store is issued.
+__global__ __launch_bounds__(256) void k_moe_hsplit(float* __restrict__ h, const uint32_t* __restrict__ hmax, int64_t groups,
+                                                    int gpr) {
+  const int64_t g = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x;
+  if (g >= groups) return;
+  const float scale = __builtin_ldexpf(1.f, -mg_row_exp(__builtin_bit_cast(float, hmax[g / gpr])));
+  float x[8];
+  f16x8 hi, lo;
+  mg_load8(h + g * 8, x);
+  mg_terms(x, scale, hi, lo);
+  f16x8* out = reinterpret_cast<f16x8*>(h + (g >> 3) * 64) + (g & 7);
+  out[0] = hi;
+  out[8] = lo;
 }
 
 // Pair counts, offsets and lists; also clears hmax. One workgroup of
@@ -155,24 +267,24 @@ __global__ __launch_bounds__(MG_T) void k_moe_group(const int32_t* __restrict__ 
 
 enum MgStage { MG_FC1_RELU = 0, MG_FC1_SWIGLU = 1, MG_FC2 = 2 };
 
-// Largest finite |v| over the 32 lanes of a lane half (lanes l, l ^ 1, ... l ^ 16).
-__device__ __forceinline__ float mg_half_max(float v) {
-#pragma unroll
-  for (int off = 16; off > 0; off >>= 1) v = fmaxf(v, __shfl_xor(v, off, 64));
-  return v;
+// v of the lane N places on in its row of 16.
+template <int N>
+__device__ __forceinline__ float mg_ror(float v) {
+  return __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, v), 0x120 + N, 0xF, 0xF, true));
 }
 
-// One 64-pair x 256-column tile of an expert's matrix; BITS-bit codes, block
+// One 128-pair x 256-column tile of an expert's matrix; BITS-bit codes, block
 // mode BKM (mg_block_mode).
 template <int ST, int BITS, int BKM>
 __global__ __launch_bounds__(MG_T, 2) void k_moe_ggemm(MoeArgs a, MgLists g, int nct) {
   constexpr bool FC2 = ST == MG_FC2;
-  constexpr int MG_STAGE = mg_stage<BITS>();
+  constexpr int SS = mg_ss<BITS>(), SB = mg_sb<BITS, BKM>();
   constexpr int BW = BITS / 4;  // dwords per fragment
   extern __shared__ __align__(16) unsigned char smem[];
-  f16* lds = reinterpret_cast<f16*>(smem);
+  f16* lds = reinterpret_cast<f16*>(smem);                                   // [2] A stages
+  uint32_t* wlds = reinterpret_cast<uint32_t*>(lds + 2 * MG_ASTAGE);         // [2] super-steps' codes
+  float* slds = reinterpret_cast<float*>(wlds + 2 * (MG_WSTAGE / 4));        // [2][SB][column] scales
   __shared__ int s_pair[MG_RT];
-  __shared__ float s_rs[MG_RT];  // 2^-e per row (staging)
   __shared__ float s_ru[MG_RT];  // 2^e per row (epilogue)
   constexpr uint32_t OOB = 0x80000000u;
   const int tid = threadIdx.x, lane = tid & 63;
@@ -193,8 +305,11 @@ __global__ __launch_bounds__(MG_T, 2) void k_moe_ggemm(MoeArgs a, MgLists g, int
     else hi = mid - 1;
   }
   const int e = lo;
-  const int lb = g.off[e] + (rt - g.toff[e]) * MG_RT;  // first list entry of the tile
-  const int nrow = min(MG_RT, g.off[e + 1] - lb);
+  // the expert's pairs over its row tiles in equal whole 32s (260 pairs: 96, 96, 68)
+  const int npe = g.off[e + 1] - g.off[e], nte = g.toff[e + 1] - g.toff[e];
+  const int rpt = ((npe + nte - 1) / nte + 31) & ~31;
+  const int lb = g.off[e] + (rt - g.toff[e]) * rpt;  // first list entry of the tile
+  const int nrow = min(rpt, g.off[e + 1] - lb);
   const int Kd = static_cast<int>(FC2 ? a.I : a.H);   // reduction length
   const int Nd = static_cast<int>(FC2 ? a.H : a.F1);  // rows of the expert matrix
   const int n0 = ct * MG_CT;
@@ -206,27 +321,13 @@ __global__ __launch_bounds__(MG_T, 2) void k_moe_ggemm(MoeArgs a, MgLists g, int
       if constexpr (FC2) ex = mg_row_exp(__builtin_bit_cast(float, g.hmax[p]));
       else ex = g.ex[p / a.k];
     }
-    s_rs[tid] = __builtin_ldexpf(1.f, -ex);
     s_ru[tid] = __builtin_ldexpf(1.f, ex);
   }
   __syncthreads();
 
-  // ---- global loads: thread t stages A row t / 8, floats 8 (t % 8) .. + 7 of
-  // the step, and 32 codes (16 bytes) of column t / 2, half t % 2. The rows
-  // belong to different tokens, so A goes through per-lane addresses (a
-  // buffer resource would have to be wave-uniform); rows past the tile's
-  // pairs repeat its first pair and their sums are never written.
-  const int arow = tid >> 3, agrp = tid & 7;
-  const int apair = s_pair[arow] < 0 ? s_pair[0] : s_pair[arow];
-  const float ascale = s_rs[arow];
-  const float* Asrc = FC2 ? a.h : a.x;
-  const float* Arow = Asrc + (FC2 ? static_cast<int64_t>(apair) * a.I : static_cast<int64_t>(apair / a.k) * a.H) + agrp * 8;
-  const int bcol = tid >> 1, bh = tid & 1;
   const uint32_t rowb = static_cast<uint32_t>(Kd) * BITS / 8u;  // bytes per expert row
   const uint8_t* Wb = FC2 ? a.fc2 + static_cast<int64_t>(e) * a.H * rowb : a.fc1 + static_cast<int64_t>(e) * a.F1 * rowb;
   const rsrc_t rB = mk_rsrc(Wb, static_cast<uint32_t>(Nd) * rowb);
-  const bool bval = n0 + bcol < Nd;
-  const uint32_t boff = bval ? static_cast<uint32_t>(n0 + bcol) * rowb : OOB;
   // this workgroup's K steps [kstep0, kstep0 + ksteps); splits of blocks of
   // 128 codes or more hold whole blocks (a split past the end holds none and
   // writes zero partials)
@@ -236,53 +337,110 @@ __global__ __launch_bounds__(MG_T, 2) void k_moe_ggemm(MoeArgs a, MgLists g, int
   const int kstep0 = sp * kper;
   const int ksteps = kall - kstep0 < kper ? kall - kstep0 : kper;
 
-  struct Regs {
-    u32x4 a[2];
-    u32x4 b[BW];
+  // ---- staging. A wave waits for its loads in the order it issued them, so the
+  // long-latency weight stream and the activations (in the L2) have waves of their
+  // own: with both in one wave every step waited for the weights loaded just before
+  // its activations (16 KB in flight per CU, 1.6 TB/s however few the pairs).
+  //  * waves 4 .. 7 (256 threads): A, one step ahead. Thread t: values 8 (t % 8) .. + 7
+  //    of rows t / 8 + 32 i (32 bytes of terms each), through per-lane addresses (the
+  //    rows belong to different tokens); rows past the tile's pairs repeat its first
+  //    pair and their sums are never written.
+  //  * waves 0 .. 3: the codes and scales, a super-step ahead. Thread t: chunk t % 8 (16
+  //    bytes) of columns t / 8 + 32 i, whole lines of eight columns per load, and the
+  //    scales of column t.
+  const int st_t = tid & 255;
+  struct ARegs {
+    u32x4 v[4][2];
   };
-  // steps past the end reload the last one (never staged)
-  auto gload = [&](Regs& r, int ks) {
-    const bool ok = ks < ksteps;
-    int kst = kstep0 + (ok ? ks : ksteps - 1);
-    kst = kst < kall - 1 ? kst : kall - 1;
-    const float* pa = Arow + kst * MG_K;
-    r.a[0] = *reinterpret_cast<const u32x4*>(pa);
-    r.a[1] = *reinterpret_cast<const u32x4*>(pa + 4);
+  const float* Arow[4];
+  {
+    const float* Asrc = FC2 ? a.h : a.yp;  // FC1: x's terms
 #pragma unroll
-    for (int i = 0; i < BW; ++i)
-      r.b[i] = bld16(rB, (ok ? boff : OOB) + static_cast<uint32_t>((kstep0 + ks) * MG_K * BITS / 8 + (bh * BW + i) * 16), 0);
-  };
-  // A: scaled, split into binary16 hi / lo in the pair order of the codes;
-  // B: the raw code dwords (dequantised when a fragment is read)
-  auto sstore = [&](const Regs& r, int stage) {
-    f16* Ah = lds + stage * MG_STAGE;
-    f16* Al = Ah + MG_RT * MG_LD;
-    uint32_t* Bw = reinterpret_cast<uint32_t*>(Al + MG_RT * MG_LD);  // [fragment][column][BW dwords]
-    f16x8 vh, vl;
-    // the eight floats by name first: this compiler folds v[i >> 2][i & 3]
-    // over an array of vectors to element 0 of each vector
-    const f32x4 lo4 = __builtin_bit_cast(f32x4, r.a[0]), hi4 = __builtin_bit_cast(f32x4, r.a[1]);
-    const float xs[8] = {lo4.x, lo4.y, lo4.z, lo4.w, hi4.x, hi4.y, hi4.z, hi4.w};
-#pragma unroll
-    for (int q = 0; q < 8; ++q) {
-      const float x = xs[(q >> 1) + 4 * (q & 1)] * ascale;  // pair order 0 4 1 5 2 6 3 7
-      const f16 h = static_cast<f16>(x);
-      vh[q] = h;
-      vl[q] = __builtin_isfinite(x) ? static_cast<f16>(x - static_cast<float>(h)) : static_cast<f16>(0.f);
+    for (int i = 0; i < 4; ++i) {
+      const int r = (st_t >> 3) + 32 * i, p = s_pair[r] < 0 ? s_pair[0] : s_pair[r];
+      Arow[i] = Asrc + (FC2 ? static_cast<int64_t>(p) * a.I : static_cast<int64_t>(p / a.k) * a.H) + (st_t & 7) * 4;
     }
-    *reinterpret_cast<f16x8*>(Ah + arow * MG_LD + agrp * 8) = vh;
-    *reinterpret_cast<f16x8*>(Al + arow * MG_LD + agrp * 8) = vl;
-    // fragment 4 bh + d of the step (codes 32 bh + 8 d .. + 7) of column bcol
-    if constexpr (BW == 1) {
+  }
+  // row tiles of 32 that hold pairs; the others are neither loaded nor read
+  const int nsub = (nrow + 31) / 32;
+  auto aload = [&](ARegs& r, int ks) {
 #pragma unroll
-      for (int d = 0; d < 4; ++d) Bw[(4 * bh + d) * MG_CT + bcol] = r.b[0][d];
-    } else {
-      // the eight dwords by name (no v[i >> 1][...] indexing, see above)
-      const u32x4 b0 = r.b[0], b1 = r.b[BW - 1];
-      const uint32_t w[8] = {b0.x, b0.y, b0.z, b0.w, b1.x, b1.y, b1.z, b1.w};
+    for (int i = 0; i < 4; ++i) {
+      if (i >= nsub) break;
+      const float* pa = Arow[i] + (kstep0 + ks) * MG_K;
+      r.v[i][0] = *reinterpret_cast<const u32x4*>(pa);
+      r.v[i][1] = *reinterpret_cast<const u32x4*>(pa + 32);
+    }
+  };
+  auto astore = [&](const ARegs& r, int stage) {
+    f16* Ah = lds + stage * MG_ASTAGE + (st_t >> 3) * MG_LD + (st_t & 7) * 8;
 #pragma unroll
-      for (int d = 0; d < 4; ++d)
-        *reinterpret_cast<u32x2*>(Bw + ((4 * bh + d) * MG_CT + bcol) * 2) = u32x2{w[2 * d], w[2 * d + 1]};
+    for (int i = 0; i < 4; ++i) {
+      if (i >= nsub) break;
+      *reinterpret_cast<u32x4*>(Ah + 32 * i * MG_LD) = r.v[i][0];
+      *reinterpret_cast<u32x4*>(Ah + (MG_RT + 32 * i) * MG_LD) = r.v[i][1];
+    }
+  };
+  // scales: [E, Nd] (row scales) or [E, Nd, Kd / block_size]
+  const int nblk = BKM ? Kd / a.bs : 1;
+  const float* S = FC2 ? a.s2 + static_cast<int64_t>(e) * a.H * nblk : a.s1 + static_cast<int64_t>(e) * a.F1 * nblk;
+  const rsrc_t rS = mk_rsrc(S, static_cast<uint32_t>(Nd) * static_cast<uint32_t>(nblk) * 4u);
+  struct WRegs {
+    u32x4 v[8];
+    uint32_t s[SB ? SB : 1];
+  };
+  // codes i0 .. i1 - 1 (of a thread's eight) of super-step u, with the first its scales;
+  // past the row: zeros
+  auto wload = [&](WRegs& r, int u, int i0, int i1) __attribute__((always_inline)) {
+    const uint32_t o = static_cast<uint32_t>((kstep0 + u * SS) * MG_K * BITS / 8 + (st_t & 7) * 16);
+    const uint32_t past = u * SS < ksteps && o < rowb ? 0u : OOB;
+#pragma unroll
+    for (int i = i0; i < i1; ++i) {
+      const int c = n0 + (st_t >> 3) + 32 * i;
+      r.v[i] = bld16(rB, ((c < Nd ? static_cast<uint32_t>(c) * rowb : OOB) | past) + o, 0);
+    }
+    if (i0 > 0) return;
+    if constexpr (SB > 0) {
+      const int c = n0 + st_t < Nd ? n0 + st_t : Nd - 1;
+      const uint32_t b = static_cast<uint32_t>((kstep0 + u * SS) * MG_K / a.bs);
+      const uint32_t so = (static_cast<uint32_t>(c) * static_cast<uint32_t>(nblk) + b) * 4u;
+      // blocks past the row's last belong to steps that are not run
+#pragma unroll
+      for (int f = 0; f < SB; f += 4) {
+        if constexpr (SB >= 4) {
+          const u32x4 v = bld16(rS, so + 4u * f, 0);
+          r.s[f] = v.x, r.s[f + 1] = v.y, r.s[f + 2] = v.z, r.s[f + 3] = v.w;
+        } else if constexpr (SB == 2) {
+          const u32x2 v = bld8(rS, so, 0);
+          r.s[0] = v.x, r.s[1] = v.y;
+        } else {
+          r.s[0] = bld_u32(rS, so, 0);
+        }
+      }
+    }
+  };
+  // codes as [fragment of the super-step][column][BW dwords], a fragment being eight
+  // codes; chunk c's columns are rotated by 8 c places, so the eight chunks a wave
+  // writes at once fall in different banks
+  auto wstore = [&](const WRegs& r, int buf) {
+    uint32_t* W = wlds + buf * (MG_WSTAGE / 4);
+    const int c = st_t & 7;
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      const int col = ((st_t >> 3) + 32 * i + 8 * c) & (MG_CT - 1);
+      const u32x4 v = r.v[i];
+      if constexpr (BW == 1) {
+        uint32_t* d = W + 4 * c * MG_CT + col;
+        d[0] = v.x, d[MG_CT] = v.y, d[2 * MG_CT] = v.z, d[3 * MG_CT] = v.w;
+      } else {
+        uint32_t* d = W + (2 * c * MG_CT + col) * 2;
+        *reinterpret_cast<u32x2*>(d) = u32x2{v.x, v.y};
+        *reinterpret_cast<u32x2*>(d + 2 * MG_CT) = u32x2{v.z, v.w};
+      }
+    }
+    if constexpr (SB > 0) {
+#pragma unroll
+      for (int f = 0; f < SB; ++f) slds[(buf * SB + f) * MG_CT + st_t] = __builtin_bit_cast(float, r.s[f]);
     }
   };
   // a fragment's eight codes -> c - 2^(bits - 1) as exact binary16, pair
@@ -291,7 +449,7 @@ __global__ __launch_bounds__(MG_T, 2) void k_moe_ggemm(MoeArgs a, MgLists g, int
   const f16x2 inv16 = {static_cast<f16>(0.0625f), static_cast<f16>(0.0625f)};
   const f16x2 n72 = {static_cast<f16>(-72.f), static_cast<f16>(-72.f)};
   const f16x2 n1152 = {static_cast<f16>(-1152.f), static_cast<f16>(-1152.f)};
-  auto dq = [&](const uint32_t* w) {
+  auto dq = [&](const uint32_t* w) __attribute__((always_inline)) {
     const uint32_t magic = 0x64006400u;
     if constexpr (BW == 1) {
       const uint32_t x = w[0], x8 = x >> 8;
@@ -312,167 +470,236 @@ __global__ __launch_bounds__(MG_T, 2) void k_moe_ggemm(MoeArgs a, MgLists g, int
     }
   };
 
-  // block sums (acc) and, with block scales, the scaled running sums (yacc)
-  f32x16 acc[2], yacc[BKM ? 2 : 1];
+  // block sums (acc) and, with block scales, the scaled running sums (yacc), of
+  // the wave's row tiles wm, wm + 2
+  f32x16 acc[2][2];
+  float yacc[BKM ? 2 : 1][BKM ? 2 : 1][16];
 #pragma unroll
-  for (int j = 0; j < 2; ++j)
-#pragma unroll
-    for (int q = 0; q < 16; ++q) acc[j][q] = 0.f;
-#pragma unroll
-  for (int j = 0; j < (BKM ? 2 : 1); ++j)
-#pragma unroll
-    for (int q = 0; q < 16; ++q) yacc[j][q] = 0.f;
-  // the scales of this lane's two columns: [E, Nd] (row scales) or
-  // [E, Nd, Kd / block_size]
-  const int nblk = BKM ? Kd / a.bs : 1;
-  const float* S = FC2 ? a.s2 + static_cast<int64_t>(e) * a.H * nblk : a.s1 + static_cast<int64_t>(e) * a.F1 * nblk;
-  int scol[2];
-#pragma unroll
-  for (int j = 0; j < 2; ++j) {
-    const int c = n0 + wn * 64 + j * 32 + (lane & 31);
-    scol[j] = (c < Nd ? c : Nd - 1) * nblk;
-  }
-  // block flushes per step: 4 / BKM inside the step, or one at its end
-  constexpr int NFL = BKM == 0 ? 0 : BKM == 8 ? 1 : 4 / BKM;
-  constexpr int NSL = NFL ? NFL : 1;
-  // (kept in place by scheduling barriers: moved among the next block's
-  // MFMAs it would hold two copies of the accumulators)
-  auto flush = [&](const float (&sc)[2]) {
-    __builtin_amdgcn_sched_barrier(0);
+  for (int i = 0; i < 2; ++i)
 #pragma unroll
     for (int j = 0; j < 2; ++j)
 #pragma unroll
       for (int q = 0; q < 16; ++q) {
-        yacc[BKM ? j : 0][q] = __builtin_fmaf(sc[j], acc[j][q], yacc[BKM ? j : 0][q]);
-        acc[j][q] = 0.f;
+        acc[i][j][q] = 0.f;
+        yacc[BKM ? i : 0][BKM ? j : 0][q] = 0.f;
+      }
+  // (kept in place by the empty asm and the scheduling barriers: sunk among the
+  // next block's MFMAs it would hold two copies of the accumulators)
+  const f32x16 zero16 = {};
+  auto flush = [&](auto na, const float (&sc)[2]) __attribute__((always_inline)) {
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int i = 0; i < na; ++i)
+#pragma unroll
+      for (int j = 0; j < 2; ++j) {
+#pragma unroll
+        for (int q = 0; q < 16; ++q) {
+          float& y = yacc[BKM ? i : 0][BKM ? j : 0][q];
+          y = __builtin_fmaf(sc[j], acc[i][j][q], y);
+          asm volatile("" : "+v"(y));
+        }
+        if constexpr (BKM == 8) acc[i][j] = zero16;
       }
     __builtin_amdgcn_sched_barrier(0);
   };
-  auto mfmas = [&](int stage, const float (&sl)[NSL][2]) {
-    const f16* Ah = lds + stage * MG_STAGE;
+  const int lcol = wn * 64 + (lane & 31);  // the lane's columns: lcol, lcol + 32
+  // step t of its super-step, on A stage `stage` and weight buffer `buf`
+  auto mfmas = [&](auto na, int stage, int buf, int t) __attribute__((always_inline)) {
+    const f16* Ah = lds + stage * MG_ASTAGE;
     const f16* Al = Ah + MG_RT * MG_LD;
-    const uint32_t* Bw = reinterpret_cast<const uint32_t*>(Al + MG_RT * MG_LD);
+    const uint32_t* W = wlds + buf * (MG_WSTAGE / 4) + 8 * t * MG_CT * BW;
+    const float* sc = slds + buf * SB * MG_CT + lcol;
 #pragma unroll
     for (int kk = 0; kk < MG_K / 16; ++kk) {
       const int ko = kk * 16 + (lane >> 5) * 8;
-      const int ar = wm * 32 + (lane & 31);
-      const f16x8 fh = *reinterpret_cast<const f16x8*>(Ah + ar * MG_LD + ko);
-      const f16x8 fl = *reinterpret_cast<const f16x8*>(Al + ar * MG_LD + ko);
+      f16x8 fh[2], fl[2];
+#pragma unroll
+      for (int i = 0; i < na; ++i) {
+        const int ar = (wm + 2 * i) * 32 + (lane & 31);
+        fh[i] = *reinterpret_cast<const f16x8*>(Ah + ar * MG_LD + ko);
+        fl[i] = *reinterpret_cast<const f16x8*>(Al + ar * MG_LD + ko);
+      }
+      const bool first = BKM >= 1 && BKM <= 4 && kk % (BKM ? BKM : 1) == 0;  // a block starts: from zero
+      const int chunk = BW == 1 ? 2 * t + kk / 2 : 4 * t + kk;  // both lane halves' fragments lie in it
 #pragma unroll
       for (int j = 0; j < 2; ++j) {
-        // codes k = ko .. ko + 7 of column wn 64 + 32 j + lane % 32: fragment ko / 8
-        const f16x8 fb = dq(Bw + ((ko >> 3) * MG_CT + wn * 64 + j * 32 + (lane & 31)) * BW);
-        acc[j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(fh, fb, acc[j], 0, 0, 0);
-        acc[j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(fl, fb, acc[j], 0, 0, 0);
+        // codes k = ko .. ko + 7 of column lcol + 32 j: fragment ko / 8
+        const f16x8 fb = dq(W + ((ko >> 3) * MG_CT + ((lcol + 32 * j + 8 * chunk) & (MG_CT - 1))) * BW);
+#pragma unroll
+        for (int i = 0; i < na; ++i) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(fh[i], fb, first ? zero16 : acc[i][j], 0, 0, 0);
+#pragma unroll
+        for (int i = 0; i < na; ++i) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(fl[i], fb, acc[i][j], 0, 0, 0);
       }
-      if constexpr (BKM >= 1 && BKM <= 4) {
-        if ((kk + 1) % BKM == 0) flush(sl[kk / BKM]);
+      if constexpr (BKM == 2 || BKM == 4) {
+        if ((kk + 1) % BKM == 0) {
+          const float* p = sc + (t * (4 / BKM) + kk / BKM) * MG_CT;
+          const float sl[2] = {p[0], p[32]};
+          flush(na, sl);
+        }
       }
     }
   };
-  // the step's block scales, loaded before its fill loads (so waiting for
-  // them never waits for the fill)
-  auto sload = [&](int ks, float (&sl)[NSL][2]) {
-    if constexpr (NFL > 0) {
-      const int kg = kstep0 + (ks < ksteps ? ks : ksteps - 1);  // in range
-#pragma unroll
-      for (int f = 0; f < NFL; ++f) {
-        const int b = BKM == 8 ? (kg * MG_K) / a.bs : kg * NFL + f;
-#pragma unroll
-        for (int j = 0; j < 2; ++j) sl[f][j] = S[scol[j] + b];
-      }
+  // Order of the K steps: column tile ct starts at super-step ct of its range and wraps
+  // around. The tiles run side by side; all at the same k, they would read the same
+  // 128 bytes of every row, whose stride of H / 2 bytes lands on few memory channels
+  // (1.6 TB/s). The start is a whole number of scale blocks.
+  const int ru = BKM == 8 && bsteps > SS ? bsteps : SS;
+  const int nru = ksteps / ru;
+  const int first_step = nru > 1 ? ct % nru * ru : 0;
+  // role 0 (waves 0 .. 3): weights; 1: activations. na: the wave's row tiles that hold
+  // pairs, 2, 1 or none (it then only stages). All loops have the same barriers.
+  auto loop = [&](auto role, auto na) __attribute__((always_inline)) {
+    ARegs ar;
+    WRegs wr;
+    int p = first_step, buf = 0;  // the step, its weight buffer
+    if constexpr (role == 0) {
+      wload(wr, p / SS, 0, 8);
+      wstore(wr, 0);
+    } else {
+      aload(ar, p);
+      astore(ar, 0);
     }
-  };
-
-  // two register sets, loads two steps ahead; double-buffered LDS, one
-  // barrier per step
-  // step ks on stage ks % 2: `nxt` holds step ks + 1 (stored to the other
-  // stage during the step), `fill` receives step ks + 2
-  auto step = [&](int ks, int stage, Regs& nxt, Regs& fill) {
-    float sl[NSL][2];
-    sload(ks, sl);
-    gload(fill, ks + 2);
-    mfmas(stage, sl);
-    if constexpr (BKM == 8) {
-      if ((kstep0 + ks + 1) % bsteps == 0) flush(sl[0]);
-    }
-    if (ks + 1 < ksteps) sstore(nxt, stage ^ 1);
     __syncthreads();
+    for (int i = 0; i < ksteps; ++i) {
+      const int t = p & (SS - 1), next = p + 1 < ksteps ? p + 1 : 0;
+      const bool last = t == SS - 1 || next == 0;  // of its super-step
+      if constexpr (role == 0) {
+        // the super-step after this one (the row's first after its last), over its first
+        // three steps (all eight at once hold up the activations' loads: 1.5 k cycles)
+        const int u = (p / SS + 1) * SS < ksteps ? p / SS + 1 : 0;
+        if constexpr (SS == 4) {
+          if (t == 0) wload(wr, u, 0, 3);
+          if (t == 1 || (last && t < 1)) wload(wr, u, 3, 6);  // the row may end inside the super-step
+          if (t == 2 || (last && t < 2)) wload(wr, u, 6, 8);
+        } else {
+          if (t == 0) wload(wr, u, 0, 8);
+        }
+      } else {
+        aload(ar, next);
+      }
+      __builtin_amdgcn_sched_barrier(0);  // the loads stay ahead of the matrix work
+      if constexpr (na > 0) {
+        mfmas(na, i & 1, buf, t);
+        if constexpr (BKM == 8) {
+          if ((kstep0 + p + 1) % bsteps == 0) {
+            const float* sp = slds + (buf * SB + (bsteps < SS ? t / bsteps : 0)) * MG_CT + lcol;
+            const float sl[2] = {sp[0], sp[32]};
+            flush(na, sl);
+          }
+        }
+      }
+      if constexpr (role == 0) {
+        if (last) wstore(wr, buf ^ 1);
+      } else {
+        astore(ar, (i + 1) & 1);
+      }
+      if (last) buf ^= 1;
+      p = next;
+      __syncthreads();
+    }
   };
   if (ksteps > 0) {  // uniform: a split past the end keeps zero sums
-    Regs r0, r1;
-    gload(r0, 0);
-    gload(r1, 1);
-    sstore(r0, 0);
-    __syncthreads();
-    int ks = 0;
-    for (; ks + 1 < ksteps; ks += 2) {
-      step(ks, 0, r1, r0);
-      step(ks + 1, 1, r0, r1);
+    const int na = ((nrow + 31) / 32 - wm + 1) / 2;
+    using I0 = std::integral_constant<int, 0>;
+    using I1 = std::integral_constant<int, 1>;
+    using I2 = std::integral_constant<int, 2>;
+    if (wm == 0) {
+      if (na >= 2) loop(I0{}, I2{});
+      else loop(I0{}, I1{});  // a tile holds a pair
+    } else {
+      if (na >= 2) loop(I1{}, I2{});
+      else if (na == 1) loop(I1{}, I1{});
+      else loop(I1{}, I0{});
     }
-    if (ks < ksteps) step(ks, 0, r1, r0);
   }
 
   // ---- epilogue: lane holds D[8 (q / 4) + 4 (lane / 32) + q % 4][lane % 32]
-  float rmax[16];
 #pragma unroll
-  for (int q = 0; q < 16; ++q) rmax[q] = 0.f;
+  for (int i = 0; i < 2; ++i) {
+    if (wm + 2 * i >= nsub) break;  // no pair in the row tile
+    const int r0 = (wm + 2 * i) * 32 + 4 * (lane >> 5);
+    auto value = [&](int j, int q, float sc) {
+      return (BKM ? yacc[BKM ? i : 0][BKM ? j : 0][q] : acc[i][j][q] * sc) * s_ru[r0 + 8 * (q >> 2) + (q & 3)];
+    };
+    float rmax[16];  // SwiGLU: even lanes' rows q, odd lanes' rows q + 1, in q / 2
 #pragma unroll
-  for (int j = 0; j < 2; ++j) {
-    const int c = n0 + wn * 64 + j * 32 + (lane & 31);
-    const float sc = BKM ? 1.f : (c < Nd ? S[c] : 0.f);
+    for (int q = 0; q < 16; ++q) rmax[q] = 0.f;
 #pragma unroll
-    for (int q = 0; q < 16; ++q) {
-      const int r = wm * 32 + 8 * (q >> 2) + 4 * (lane >> 5) + (q & 3);
-      const int p = s_pair[r];
-      const float v = (BKM ? yacc[BKM ? j : 0][q] : acc[j][q] * sc) * s_ru[r];
-      if constexpr (FC2) {
-        if (p >= 0 && c < Nd) a.yp[(static_cast<int64_t>(p) * ks2 + sp) * a.H + c] = v;
-      } else if constexpr (ST == MG_FC1_SWIGLU) {
-        // gate = row 2m (even lane), linear = row 2m + 1 (odd lane)
-        const float other = __shfl_xor(v, 1, 64);
-        const float o = swiglu(v, other, a);
-        if ((lane & 1) == 0 && p >= 0 && c < Nd) {
-          a.h[static_cast<int64_t>(p) * a.I + c / 2] = o;
-          if (__builtin_isfinite(o)) rmax[q] = fmaxf(rmax[q], __builtin_fabsf(o));
+    for (int j = 0; j < 2; ++j) {
+      const int c = n0 + wn * 64 + j * 32 + (lane & 31);
+      const float sc = BKM ? 1.f : (c < Nd ? S[c] : 0.f);
+      if constexpr (ST == MG_FC1_SWIGLU) {
+        // gate = FC1 row 2m (even lane), linear = row 2m + 1 (odd lane): of two output
+        // rows the even lane forms the first, the odd lane the second
+        const bool odd = lane & 1;
+#pragma unroll
+        for (int q = 0; q < 16; q += 2) {
+          const float v0 = value(j, q, sc), v1 = value(j, q + 1, sc);
+          const float other = __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, odd ? v0 : v1), 0xB1, 0xF, 0xF, true));
+          const float o = swiglu(odd ? other : v0, odd ? v1 : other, a);
+          const int p = s_pair[r0 + 8 * (q >> 2) + (q & 3) + (odd ? 1 : 0)];
+          if (p >= 0 && c < Nd) {
+            a.h[static_cast<int64_t>(p) * a.I + c / 2] = o;
+            if (__builtin_isfinite(o)) rmax[q >> 1] = fmaxf(rmax[q >> 1], __builtin_fabsf(o));
+          }
         }
       } else {
-        const float o = fmaxf(v, 0.f);
-        if (p >= 0 && c < Nd) {
-          a.h[static_cast<int64_t>(p) * a.I + c] = o;
-          if (__builtin_isfinite(o)) rmax[q] = fmaxf(rmax[q], o);
+#pragma unroll
+        for (int q = 0; q < 16; ++q) {
+          const int p = s_pair[r0 + 8 * (q >> 2) + (q & 3)];
+          const float v = value(j, q, sc);
+          if constexpr (FC2) {
+            if (p >= 0 && c < Nd) a.yp[(static_cast<int64_t>(p) * ks2 + sp) * a.H + c] = v;
+          } else {
+            const float o = fmaxf(v, 0.f);
+            if (p >= 0 && c < Nd) {
+              a.h[static_cast<int64_t>(p) * a.I + c] = o;
+              if (__builtin_isfinite(o)) rmax[q] = fmaxf(rmax[q], o);
+            }
+          }
         }
       }
     }
-  }
-  if constexpr (!FC2) {
-    // each row's largest |h| over this tile, into the pair's running maximum
-    // (non-negative floats order like their bit patterns)
+    if constexpr (!FC2) {
+      // each row's largest |h| over this tile, into the pair's running maximum
+      // (non-negative floats order like their bit patterns)
+      constexpr bool SW = ST == MG_FC1_SWIGLU;
 #pragma unroll
-    for (int q = 0; q < 16; ++q) {
-      const float m = mg_half_max(rmax[q]);
-      const int r = wm * 32 + 8 * (q >> 2) + 4 * (lane >> 5) + (q & 3);
-      const int p = s_pair[r];
-      if ((lane & 31) == 0 && p >= 0 && m > 0.f) atomicMax(g.hmax + p, __builtin_bit_cast(uint32_t, m));
+      for (int q = 0; q < (SW ? 8 : 16); ++q) {
+        float m = rmax[q];
+        if constexpr (!SW) m = fmaxf(m, mg_ror<1>(m));
+        m = fmaxf(m, mg_ror<2>(m));
+        m = fmaxf(m, mg_ror<4>(m));
+        m = fmaxf(m, mg_ror<8>(m));
+        m = fmaxf(m, __shfl_xor(m, 16, 64));
+        const int qq = SW ? 2 * q + (lane & 1) : q;
+        const int p = s_pair[r0 + 8 * (qq >> 2) + (qq & 3)];
+        if ((lane & 31) < (SW ? 2 : 1) && p >= 0 && m > 0.f) atomicMax(g.hmax + p, __builtin_bit_cast(uint32_t, m));
+      }
     }
   }
 }
 
 // y[t][n] = sum over slots s of w[t k + s] * yp[t k + s][n], in slot order,
-// each slot's a.ks FC2 splits summed first in split order.
+// each slot's a.ks FC2 splits summed first in split order; four columns per
+// thread (H % 64 == 0).
 __global__ __launch_bounds__(256) void k_moe_combine(MoeArgs a) {
   const int64_t i = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x;
-  if (i >= a.T * a.H) return;
-  const int64_t t = i / a.H, n = i % a.H;
-  float y = 0.f;
+  const int64_t h4 = a.H / 4;
+  if (i >= a.T * h4) return;
+  const int64_t t = i / h4, n = i % h4 * 4;
+  f32x4 y = {0.f, 0.f, 0.f, 0.f};
   for (int s = 0; s < a.k; ++s) {
     const int64_t pair = t * a.k + s;
     const float* part = a.yp + pair * a.ks * a.H + n;
-    float v = part[0];
-    for (int sp = 1; sp < a.ks; ++sp) v += part[static_cast<int64_t>(sp) * a.H];
-    y = __builtin_fmaf(a.wts[pair], v, y);
+    f32x4 v = *reinterpret_cast<const f32x4*>(part);
+    for (int sp = 1; sp < a.ks; ++sp) v += *reinterpret_cast<const f32x4*>(part + static_cast<int64_t>(sp) * a.H);
+    const float w = a.wts[pair];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) y[e] = __builtin_fmaf(w, v[e], y[e]);
   }
-  a.y[i] = y;
+  typedef f32x4 f32x4_a4 __attribute__((aligned(4)));  // y need not be 16-byte aligned
+  *reinterpret_cast<f32x4_a4*>(a.y + t * a.H + n) = y;
 }
 
 }  // namespace
