@@ -11,6 +11,7 @@ import os
 import shutil
 import subprocess
 import sys
+import sysconfig
 from concurrent.futures import ThreadPoolExecutor
 
 HERE = os.path.dirname(os.path.abspath(__file__))
@@ -19,6 +20,7 @@ CSRC = os.path.join(HERE, "csrc")
 OBJ_DIR = os.path.join(HERE, "_build")
 LIB_DIR = os.path.join(HERE, "lib")
 LIB = os.path.join(LIB_DIR, "libxrmm.so")
+FRONT = os.path.join(LIB_DIR, "_xrmm_torch.so")  # native front end of ops.py (CPython extension)
 RUNNER = os.path.join(LIB_DIR, "xrmm_execute")  # job-JSON runner over the C ABI
 ARCH = os.environ.get("XRMM_OFFLOAD_ARCH", "gfx950")
 
@@ -85,6 +87,19 @@ def _run(cmd, verbose):
         sys.stderr.write("\n".join(noise) + "\n")
 
 
+def build_front(cxx, verbose):
+    """The torch extension: host code against the installed torch's headers."""
+    import torch
+    t = os.path.dirname(torch.__file__)
+    inc = [os.path.join(t, "include"), os.path.join(t, "include", "torch", "csrc", "api", "include"),
+           sysconfig.get_paths()["include"]]
+    _run([cxx, "-O2", "-std=c++17", "-fPIC", "-shared", "-Wall", "-Wno-maybe-uninitialized",
+          f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}", *[a for i in inc for a in ("-I", i)],
+          os.path.join(CSRC, "xrmm_torch.cpp"), "-o", FRONT + ".tmp", "-L", os.path.join(t, "lib"), "-ltorch_python",
+          "-ltorch_cpu", "-lc10"], verbose)
+    os.replace(FRONT + ".tmp", FRONT)
+
+
 def build(verbose: bool = False, jobs: int | None = None) -> str:
     os.makedirs(LIB_DIR, exist_ok=True)
     os.makedirs(OBJ_DIR, exist_ok=True)
@@ -105,6 +120,7 @@ def build(verbose: bool = False, jobs: int | None = None) -> str:
     _run([cxx, "-O2", "-std=c++17", "-Wall", "-I", os.path.join(ROOT, "include"), os.path.join(CSRC, "xrmm_execute.cpp"),
           "-L", LIB_DIR, "-lxrmm", "-Wl,-rpath,$ORIGIN", "-o", RUNNER + ".tmp"], verbose)
     os.replace(RUNNER + ".tmp", RUNNER)
+    build_front(cxx, verbose)
     return LIB
 
 

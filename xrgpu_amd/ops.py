@@ -12,6 +12,11 @@ float zero points ``[N, ceil(K/bs)]`` or packed uint8 zero points
 """
 from __future__ import annotations
 
+import ctypes
+import importlib.util
+import os
+import warnings
+
 import torch
 
 from . import _native as nat
@@ -34,6 +39,40 @@ def _stream(stream=None, device=None):
     if _raw_stream is not None:
         return _raw_stream(device if device is not None and device >= 0 else torch.cuda.current_device())
     return torch.cuda.current_stream().cuda_stream
+
+
+# The native front end (csrc/xrmm_torch.cpp): None until first asked for, False where it
+# is not built, built for another torch, or there is no GPU. Its functions return None for whatever they do not
+# take, and the checks below then decide.
+_FRONT = None
+
+
+def _front():
+    global _FRONT
+    if _FRONT is None:
+        _FRONT = _load_front()
+    return _FRONT
+
+
+def _load_front():
+    path = os.path.join(os.path.dirname(os.path.abspath(__file__)), "lib", "_xrmm_torch.so")
+    if _raw_stream is None or not os.path.exists(path) or not torch.cuda.is_available():
+        return False
+    spec = importlib.util.spec_from_file_location("_xrmm_torch", path)
+    try:
+        mod = importlib.util.module_from_spec(spec)
+        spec.loader.exec_module(mod)
+        same = torch.__version__.split("+")[0] == mod.torch_version.split("+")[0]
+    except ImportError:  # symbols of another torch
+        same = False
+    if not same:
+        warnings.warn("xrgpu_amd/lib/_xrmm_torch.so was built for another torch; run `python -m xrgpu_amd.build`")
+        return False
+    lib = nat.lib()
+    mod.bind(_raw_stream, nat.check, *(ctypes.cast(getattr(lib, n), ctypes.c_void_p).value for n in (
+        "xrmm_matmul_nbits", "xrmm_matmul_nbits_workspace_bytes", "xrmm_matmul_nbits_fused_workspace_bytes",
+        "xrmm_matmul_nbits_qkv_ws", "xrmm_matmul_nbits_mlp_ws", "xrmm_matmul_bnb4", "xrmm_gather_block_quantized")))
+    return mod
 
 
 def _check_dev(*ts):
@@ -130,6 +169,10 @@ def matmul_nbits(A, B, scales, zero_points=None, bias=None, *, K=None, N=None, b
     need different workspaces. Under HIP graph capture without a caller
     workspace the call runs unsplit, so a captured graph never depends on a
     workspace this module might replace or share with another graph."""
+    if out is None and workspace is None and stream is None and _front():
+        y = _FRONT.matmul(A, B, scales, zero_points, bias, K, N, bits, block_size)
+        if y is not None:
+            return y
     K = int(K if K is not None else A.shape[-1])
     N = int(N if N is not None else B.shape[0])
     if A.shape[-1] != K:
@@ -275,6 +318,11 @@ def matmul_nbits_qkv(A, q_B, q_scales, k_B, k_scales, v_B, v_scales, *, norm_sca
     Prefill geometries normalise the rows once into a workspace
     (``fused_workspace_bytes``); pass ``workspace`` to supply it, else one is
     taken from torch's caching allocator."""
+    if workspace is None and stream is None and _front():
+        r = _FRONT.qkv(A, q_B, q_scales, k_B, k_scales, v_B, v_scales, norm_scale, skip, K, Nq, Nkv, bits, block_size,
+                       epsilon, q_zero_points, k_zero_points, v_zero_points, want_residual)
+        if r is not None:
+            return r
     K = int(K if K is not None else A.shape[-1])
     Nq = int(Nq if Nq is not None else q_B.shape[0])
     Nkv = int(Nkv if Nkv is not None else k_B.shape[0])
@@ -314,6 +362,11 @@ def matmul_nbits_mlp(A, gate_B, gate_scales, up_B, up_scales, *, skip=None, norm
     Prefill geometries with skip or norm_scale normalise the rows once into a
     workspace (``fused_workspace_bytes``); pass ``workspace`` to supply it,
     else one is taken from torch's caching allocator."""
+    if workspace is None and stream is None and activation in nat.ACT and _front():
+        r = _FRONT.mlp(A, gate_B, gate_scales, up_B, up_scales, skip, norm_scale, gate_bias, up_bias, K, N, bits,
+                       block_size, epsilon, nat.ACT[activation], gate_zero_points, up_zero_points, want_residual)
+        if r is not None:
+            return r
     K = int(K if K is not None else A.shape[-1])
     N = int(N if N is not None else gate_B.shape[0])
     if activation not in nat.ACT:
@@ -435,6 +488,10 @@ def gather_block_quantized(data, indices, scales, zero_points=None, *, bits=4, b
     stream and raises ``XrmmError`` ("GPU operator contract validation failed:
     code 55") as the reference's run does.
     """
+    if status is not None and not check and stream is None and _front():
+        r = _FRONT.gather(data, indices, scales, zero_points, status, bits, block_size)
+        if r is not None:
+            return r
     if status is not None and (status.dtype not in (torch.int32, torch.uint32) or status.numel() < 1):
         raise nat.XrmmInvalid("status must be an int32 or uint32 tensor of at least one element")
     if data.dtype != torch.uint8 or (zero_points is not None and zero_points.dtype != torch.uint8):
@@ -473,6 +530,10 @@ def matmul_bnb4(A, B, absmax, *, K, N, block_size=32, quant_type=1, trans_b=1, o
     A ``[M, K]`` float32/float16, B uint8 ``ceil(N*K/2)`` bytes (even flat index
     in the high nibble), absmax ``ceil(N*K/block_size)`` in A's dtype.
     """
+    if out is None and stream is None and _front():
+        y = _FRONT.bnb4(A, B, absmax, K, N, block_size, quant_type, trans_b)
+        if y is not None:
+            return y
     if A.dtype not in _T1 or absmax.dtype != A.dtype:
         raise nat.XrmmInvalid("Logical dtype outside frozen contract: aT")
     if B.dtype != torch.uint8:
