@@ -15,7 +15,8 @@ its exact rounding is unknown; this oracle fixes one:
 
 * per row and block of 128 activations: ``scale = float32(max|a|) / 127``
   (float32), ``q = rint(a / scale)`` (float32 division, round half to even,
-  within [-127, 127]); a block of zeros has scale 0 and codes 0;
+  within [-127, 127]); a block of zeros has scale 0 and codes 0, a block that
+  holds an infinity or NaN the scale NaN (its row's results are NaN) and codes 0;
 * ``Y[m, n] = sum over blocks of scale[m, b] * sum_k q[m, k] * W[n, k]`` with
   the reference's float32 ``W`` (``oracle.dequantize``), float64 sums, one
   rounding to A's dtype (+ bias).
@@ -40,10 +41,11 @@ def quantize_activations(A, K: int):
     M = x.shape[0]
     blocks = x.reshape(M, K // QBLOCK, QBLOCK)
     amax = np.abs(blocks).max(axis=2) if M else np.zeros((0, K // QBLOCK), np.float32)
-    scale = (amax.astype(np.float32) / np.float32(127)).astype(np.float32)
-    safe = np.where(scale == 0, np.float32(1), scale)
-    q = np.rint((blocks / safe[:, :, None]).astype(np.float32))
-    q = np.where(scale[:, :, None] == 0, 0, np.clip(q, -127, 127)).astype(np.int8)
+    finite = np.isfinite(amax)
+    scale = np.where(finite, amax / np.float32(127), np.float32(np.nan)).astype(np.float32)
+    coded = finite & (scale != 0)
+    q = np.rint((np.where(coded[:, :, None], blocks, 0) / np.where(coded, scale, np.float32(1))[:, :, None]).astype(np.float32))
+    q = np.clip(q, -127, 127).astype(np.int8)
     return q.reshape(M, K), scale
 
 

@@ -103,3 +103,29 @@ def test_int8a(gpu, M, K, N, bs, zp, bias, dt):
     W = O.dequantize(B, S, Z, K, 4, bs, kind).astype(np.float64)
     mag = np.abs(q.astype(np.float64) * np.repeat(sa.astype(np.float64), 128, 1)) @ np.abs(W).T
     close(got, ref, mag, K // 16, dt == np.float16)  # block sums are exact: a few roundings per block
+
+
+@pytest.mark.parametrize("M", [7, 520])  # the GEMV, the GEMM (2^28 multiply-adds)
+@pytest.mark.parametrize("bs,dt", [(32, np.float16), (128, np.float32)])
+def test_int8a_nonfinite(gpu, M, bs, dt):
+    """A block of 128 activations that holds an infinity or NaN has no scale: its row is
+    NaN, as in the oracle (Inf times the other codes' zero), whatever the row count;
+    the other rows are what they are without it."""
+    K, N = 1024, 520
+    assert (M >= 8 and M * K * N >= 1 << 28) == (M == 520)
+    rng = np.random.default_rng(M + bs)
+    A = rng.standard_normal((M, K)).astype(dt)
+    B = rng.integers(0, 256, (N, K // bs, bs // 2), dtype=np.uint8)
+    S = rng.uniform(0.005, 0.05, (N, K // bs)).astype(dt)
+    bad = {0: (5, np.inf), 2: (700, -np.inf), 3: (130, np.nan), M - 1: (1023, np.inf)}
+    clean = ops().matmul_nbits_int8a(dev(A), dev(B), dev(S), K=K, N=N, block_size=bs).cpu().numpy()
+    A[2, 701] = np.inf
+    for m, (k, v) in bad.items():
+        A[m, k] = v
+    A[1, 0:128:32] = np.inf  # one in every chunk of 32
+    got = ops().matmul_nbits_int8a(dev(A), dev(B), dev(S), K=K, N=N, block_size=bs).cpu().numpy()
+    rows = sorted({1, *bad})
+    ref = Q8.matmul_nbits_int8a(A[rows], B, S, None, None, K=K, N=N, block_size=bs, zp_kind=None)
+    assert np.isnan(ref).all() and np.isnan(got[rows]).all()
+    rest = np.setdiff1d(np.arange(M), rows)
+    assert np.array_equal(got[rest], clean[rest])

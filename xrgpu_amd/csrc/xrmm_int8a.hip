@@ -5,7 +5,10 @@
 // 1. k_i8a_quant: one wave per (row, block of 128 activations): scale =
 //    max|a| / 127, codes rint(a / scale) (float32, round half to even), the
 //    codes of each group of 8 stored as k0 k2 k4 k6 k1 k3 k5 k7 so that they
-//    line up with the low and high nibbles of a weight dword.
+//    line up with the low and high nibbles of a weight dword. A block that holds
+//    an infinity or NaN has the scale NaN: Inf times the other codes' zero is
+//    NaN in every order of summation, and both consumers then agree whatever
+//    part of the block they add before they scale.
 // 2. k_i8a_gemv: one wave per output column; its lanes split K into chunks of
 //    32 codes, convert the column's codes once to signed bytes (code - zero:
 //    (c | 0x80) - z, then ^ 0x80, per byte without borrows), and for each row
@@ -36,7 +39,8 @@ __global__ __launch_bounds__(I8T) void k_i8a_quant(Int8aArgs a) {
   float mx = fmaxf(fabsf(x0), fabsf(x1));
 #pragma unroll
   for (int off = 32; off > 0; off >>= 1) mx = fmaxf(mx, __shfl_xor(mx, off, 64));
-  const float scale = __fdiv_rn(mx, 127.f);
+  const bool finite = __builtin_isfinite(x0) && __builtin_isfinite(x1);  // fmaxf passes over NaN
+  const float scale = __builtin_amdgcn_ballot_w64(!finite) != 0 ? __builtin_nanf("") : __fdiv_rn(mx, 127.f);
   auto code = [&](float x) -> int8_t {
     if (scale == 0.f) return 0;
     const float q = rintf(__fdiv_rn(x, scale));
