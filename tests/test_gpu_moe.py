@@ -258,3 +258,26 @@ def test_grouped_nonfinite_rows(gpu):
     assert not np.isfinite(ref[3]).all() and not np.isfinite(ref[7]).all()
     ok, err, lim = O.tolerance_ok(got, ref, np.float32)
     assert ok, f"max|d|={err} > {lim}"
+
+
+@pytest.mark.parametrize("act,scale", [("relu", 1e-36), ("swiglu", 1e-18)])  # x tiny; only h = gate * lin / 2 tiny
+@pytest.mark.parametrize("bs", [0, 64])
+def test_grouped_tiny_rows(gpu, act, scale, bs):
+    """A token whose activations (or their products) are near the smallest float32 values
+    keeps finite, accurate outputs, and the other tokens' outputs do not change."""
+    T, H, I, E = 40, 128, 192, 4
+    rng = np.random.default_rng(17)
+    sw = act == "swiglu"
+    i = rand_case(rng, T, H, I, E, 4, bs, sw)
+    at = dict(k=2, activation=act, swiglu_fusion=1 if sw else 0, bits=4, block_size=bs, alpha=1.0, beta=0.0,
+              swiglu_limit=None)
+    assert ops().qmoe_kernel(T, H, E, 2 * I if sw else I, 2, 4, bs, act, 1 if sw else 0) == "qmoe_grouped"
+    clean = run_gpu(i, at)
+    i["inputT"][3] *= np.float32(scale)
+    i["inputT"][9] = 0
+    got, ref = run_gpu(i, at), run_oracle(i, at)
+    keep = np.setdiff1d(np.arange(T), [3, 9])
+    assert np.array_equal(got[keep], clean[keep])
+    assert np.all(got[9] == 0)
+    ok, err, lim = O.tolerance_ok(got[3], ref[3], np.float32)
+    assert ok and np.isfinite(got[3]).all() and np.abs(ref[3]).max() > 0, (err, lim)

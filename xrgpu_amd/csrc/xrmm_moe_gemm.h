@@ -92,13 +92,14 @@ struct MgLists {
   int32_t* ex;     // [T] row exponent of x
 };
 
-// Exponent e such that |v| * 2^-e is near 2^14 for the row maximum v
-// (0 for an all-zero row).
+// Exponent e such that |v| * 2^-e is near 2^14 for the row maximum v (0 for an
+// all-zero row), at least -126 so that 2^e and 2^-e are both normal float32
+// values (rows below 2^-112 keep fewer bits).
 __device__ __forceinline__ int mg_row_exp(float mx) {
   if (!(mx > 0.f) || !__builtin_isfinite(mx)) return 0;
   int e = 0;
   (void)__builtin_frexpf(mx, &e);  // mx = f * 2^e, f in [0.5, 1)
-  return e - 15;
+  return e - 15 < -126 ? -126 : e - 15;
 }
 
 // Eight values times 2^-e as their binary16 terms, hi then lo, in the codes' pair
