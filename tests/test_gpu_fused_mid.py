@@ -82,3 +82,17 @@ def test_mlp(gpu, M, K, N, Nkv, bs, zp, skip):
     ref = h[0] / (1 + np.exp(-h[0])) * h[1]
     ok, err, lim = O.tolerance_ok(y.cpu().numpy(), ref.astype(np.float16), np.float16)
     assert ok, (err, lim)
+
+
+def test_two_gib_of_activations(gpu):
+    """Activations that end 32 bytes below 2^31: the K groups' step past the last row
+    reads zeros, not the first row's infinities."""
+    M, K, N, bs = 8191, 131088, 8, 32
+    rng = np.random.default_rng(4)
+    g, u = ([dev(t) for t in weights(rng, N, K, bs, None)[:2]] for _ in range(2))
+    A = torch.zeros((M, K), dtype=torch.float16, device="cuda")
+    A[:2] = float("inf")
+    A[-70:] = torch.randn(70, K, device="cuda", generator=torch.Generator("cuda").manual_seed(2)).half()
+    y, _ = ops().matmul_nbits_mlp(A, *g, *u, block_size=bs)
+    want, _ = ops().matmul_nbits_mlp(A[-70:].contiguous(), *g, *u, block_size=bs)
+    assert torch.equal(y[-70:], want) and torch.isfinite(want).all()

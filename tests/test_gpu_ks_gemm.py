@@ -129,3 +129,19 @@ def test_int8a_nonfinite(gpu, M, bs, dt):
     assert np.isnan(ref).all() and np.isnan(got[rows]).all()
     rest = np.setdiff1d(np.arange(M), rows)
     assert np.array_equal(got[rest], clean[rest])
+
+
+def test_bnb4_two_gib_of_activations(gpu):
+    """Activations that end just below 2^31 bytes: the steps past the last row's K read
+    zeros, not the first rows (whose infinities would reach the last row)."""
+    M, K, N, bs = (1 << 25) - 1, 32, 8, 32
+    rng = np.random.default_rng(1)
+    b = dev(rng.integers(0, 256, N * K // 2, dtype=np.uint8))
+    s = dev(rng.uniform(0.1, 1, N).astype(np.float16))
+    A = torch.zeros((M, K), dtype=torch.float16, device="cuda")
+    A[:64] = float("inf")
+    A[-8:] = torch.randn(8, K, device="cuda", generator=torch.Generator("cuda").manual_seed(2)).half()
+    assert ops().bnb4_kernel(M, K, N, bs, 1, 1, torch.float16) == "bnb4_gemm"
+    y = ops().matmul_bnb4(A, b, s, K=K, N=N, block_size=bs)
+    assert torch.equal(y[-8:], ops().matmul_bnb4(A[-8:].contiguous(), b, s, K=K, N=N, block_size=bs))
+    assert torch.isfinite(y[64:]).all()

@@ -125,13 +125,15 @@ __global__ __launch_bounds__(THREADS, 2) void k_gemm_ks(Args a) {
   const uint32_t nas = static_cast<uint32_t>(K) / 128u;
   const rsrc_t rAs = mk_rsrc(Q8 ? static_cast<const void*>(a.as) : a.A, Q8 ? static_cast<uint32_t>(a.M) * nas * 4u : 0u);
   const uint32_t asoff = gt < RT && m0 + gt < a.M ? static_cast<uint32_t>(m0 + gt) * nas * 4u : OOB;
+  // (the bound is set in the sum: set in the offset, a sum past 2^31 would wrap to the
+  // first rows)
   auto aload = [&](ARegs& r, int s) {
     const uint32_t k = static_cast<uint32_t>(k0 + s) * KSTEP;
     const uint32_t past = s < n && k + static_cast<uint32_t>(grp) * 8u < static_cast<uint32_t>(K) ? 0u : OOB;  // K % 32 == 0: whole pieces
 #pragma unroll
     for (int i = 0; i < AP; ++i) {
-      if constexpr (Q8) r.q[i] = bld8(rA, (aoff[i] | past) + k * ES, 0);
-      else r.h[i] = bld16(rA, (aoff[i] | past) + k * ES, 0);
+      if constexpr (Q8) r.q[i] = bld8(rA, (aoff[i] + k * ES) | past, 0);
+      else r.h[i] = bld16(rA, (aoff[i] + k * ES) | past, 0);
     }
     if constexpr (Q8) r.as = __builtin_bit_cast(float, bld_u32(rAs, (asoff | (s < n ? 0u : OOB)) + k / 128u * 4u, 0));
   };

@@ -113,7 +113,7 @@ __global__ __launch_bounds__(THREADS * kgroups(WIDE), WIDE ? 2 : 4) void k_gemm_
     const uint32_t k = static_cast<uint32_t>(ks0 + ks) * BK;
     const uint32_t apast = k + static_cast<uint32_t>(grp) * 8u < static_cast<uint32_t>(K) ? 0u : OOB;  // K % 8 == 0
 #pragma unroll
-    for (int i = 0; i < 2; ++i) r.a[i] = bld16(rA, (aoff[i] | apast) + k * 2u, 0);
+    for (int i = 0; i < 2; ++i) r.a[i] = bld16(rA, (aoff[i] + k * 2u) | apast, 0);
     const uint32_t o = k / 2u;
     const uint32_t past = none | (o + static_cast<uint32_t>(bq * DP * 4) < rowb ? 0u : OOB);
     if constexpr (DP == 4) {
