@@ -177,3 +177,25 @@ def test_splitk_geometries_under_graph_capture(gpu, caller_workspace):
             y = ops().matmul_nbits(A, B, S, Z, b, block_size=bs)
             torch.cuda.synchronize()
             _check(y, *cases[1 - i], K, N, bs)
+
+
+def test_two_gib_of_activations(gpu):
+    """Activations that end 32 bytes below 2^31, without a workspace (two K groups of an
+    odd number of steps): the step past the last row reads zeros, not the first rows."""
+    from xrgpu_amd import _native as nat
+    M, K, N, bs = 8191, 131088, 8, 32
+    rng = np.random.default_rng(4)
+    B, S = dev(rng.integers(0, 256, (N, O.k_blocks(K, bs), bs // 2), dtype=np.uint8)), dev(
+        rng.uniform(0.001, 0.02, (N, O.k_blocks(K, bs))).astype(np.float16))
+    A = torch.zeros((M, K), dtype=torch.float16, device="cuda")
+    A[:2] = float("inf")
+    A[-70:] = torch.randn(70, K, device="cuda", generator=torch.Generator("cuda").manual_seed(2)).half()
+    last = A[-70:].contiguous()
+    out = []
+    for a in (A, last):
+        Y = torch.empty((a.shape[0], N), dtype=torch.float16, device="cuda")
+        nat.check(nat.lib().xrmm_matmul_nbits(a.data_ptr(), B.data_ptr(), S.data_ptr(), None, nat.UNSPECIFIED, None,
+                                              Y.data_ptr(), a.shape[0], K, N, 4, bs, nat.F16,
+                                              torch.cuda.current_stream().cuda_stream))
+        out.append(Y[-70:])
+    assert torch.equal(*out) and torch.isfinite(out[1]).all()

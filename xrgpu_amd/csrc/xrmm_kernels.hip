@@ -216,7 +216,7 @@ __global__ __launch_bounds__(256 * KG) void k_gemm_q4(Launch L) {
     const uint32_t kpast = (k < K32 && kt < kend) ? 0u : OOB;  // K % 8 == 0: groups are whole
 #pragma unroll
     for (int i = 0; i < 4; ++i)
-      r.a[i] = __builtin_bit_cast(f16x8, bld16(rA, (aoff[i] | kpast) + static_cast<uint32_t>(kt) * (GM_BK * 2), 0));
+      r.a[i] = __builtin_bit_cast(f16x8, bld16(rA, (aoff[i] + static_cast<uint32_t>(kt) * (GM_BK * 2)) | kpast, 0));
     const uint32_t ch = static_cast<uint32_t>(kt) * 2u + static_cast<uint32_t>(bh);
     const uint32_t past = (ch < static_cast<uint32_t>(nchunk) && kt < kend) ? 0u : OOB;
     r.b = bld16(rB, (bcol_off | past) + ch * 16u, 0);
