@@ -145,3 +145,43 @@ def test_bnb4_two_gib_of_activations(gpu):
     y = ops().matmul_bnb4(A, b, s, K=K, N=N, block_size=bs)
     assert torch.equal(y[-8:], ops().matmul_bnb4(A[-8:].contiguous(), b, s, K=K, N=N, block_size=bs))
     assert torch.isfinite(y[64:]).all()
+
+
+def off(a, items=1):
+    """a on the GPU, contiguous, its data `items` elements past an allocation's start."""
+    buf = torch.zeros(a.size + items, dtype=dev(a).dtype, device="cuda")
+    buf[items:] = dev(a).flatten()
+    return buf[items:].view(a.shape)
+
+
+@pytest.mark.parametrize("bs", [32, 64])
+def test_bnb4_unaligned_absmax(gpu, bs):
+    """absmax two bytes past a word (the GEMM's word loads would be misaligned): the GEMV's
+    results, row for row."""
+    M, K, N = 9, 256, 96
+    rng = np.random.default_rng(bs)
+    a = dev(rng.standard_normal((M, K)).astype(np.float16))
+    b = dev(rng.integers(0, 256, N * K // 2, dtype=np.uint8))
+    s = rng.uniform(0.02, 1.5, N * K // bs).astype(np.float16)
+    kw = dict(K=K, N=N, block_size=bs)
+    got = ops().matmul_bnb4(a, b, off(s), **kw)
+    # the same four-row passes, by calls of four rows (aligned absmax)
+    want = torch.cat([ops().matmul_bnb4(torch.cat([a[m:m + 4], a[:4]])[:4].contiguous(), b, dev(s), **kw)[:M - m]
+                      for m in range(0, M, 4)])
+    assert torch.equal(got, want)
+
+
+@pytest.mark.parametrize("which", ["scales", "zero_points"])
+def test_int8a_unaligned_metadata(gpu, which):
+    """Scales at an odd element or zero points at an odd byte: the GEMV's results."""
+    M, K, N, bs = 264, 1024, 1000, 32
+    assert M * K * N >= 1 << 28
+    rng = np.random.default_rng(5)
+    A = dev(rng.standard_normal((M, K)).astype(np.float16))
+    B = dev(rng.integers(0, 256, (N, K // bs, bs // 2), dtype=np.uint8))
+    S = rng.uniform(0.005, 0.05, (N, K // bs)).astype(np.float16)
+    Z = rng.integers(0, 256, (N, K // bs // 2), dtype=np.uint8)
+    kw = dict(K=K, N=N, block_size=bs)
+    got = ops().matmul_nbits_int8a(A, B, off(S) if which == "scales" else dev(S), off(Z) if which == "zero_points" else dev(Z), **kw)
+    want = torch.cat([ops().matmul_nbits_int8a(A[m:m + 6].contiguous(), B, dev(S), dev(Z), **kw) for m in range(0, M, 6)])
+    assert torch.equal(got, want)

@@ -41,7 +41,12 @@ Planes planes(const float (&book)[16]) {
 
 bool bnb4_gemm_ok(const Bnb4Args& a) {
   if (!a.f16 || !a.tb || (a.M < kBnb4GemmMinM && bnb4_fast_ok(a)) || a.K % 32 != 0 || a.bs < 32 || (a.bs & (a.bs - 1)) != 0 || a.K % a.bs != 0) return false;
-  if ((reinterpret_cast<uintptr_t>(a.B) & 15) != 0 || (reinterpret_cast<uintptr_t>(a.A) & 15) != 0) return false;
+  // 16-byte loads of A and B; a column's block scales load as 4- and 8-byte words,
+  // which want absmax on a word (a view at an odd element stays with the GEMV, which
+  // loads them one by one)
+  if ((reinterpret_cast<uintptr_t>(a.B) & 15) != 0 || (reinterpret_cast<uintptr_t>(a.A) & 15) != 0 ||
+      (reinterpret_cast<uintptr_t>(a.absmax) & 3) != 0)
+    return false;
   // 32-bit buffer ranges, row and grid counts
   const int64_t lim = int64_t(1) << 31;
   return a.N * (a.K / 2) < lim && a.M * a.K * 2 < lim && a.M < lim / 2 && (a.M + 31) / 32 * ((a.N + 31) / 32) < lim;

@@ -6,6 +6,9 @@
 namespace xrmm {
 
 bool i8a_gemm_ok(const Int8aArgs& a) {
+  // scales load as words of 4 to 16 bytes, zero points as 2 bytes (the GEMV loads both
+  // one by one and keeps views at odd elements)
+  if ((reinterpret_cast<uintptr_t>(a.S) & 3) != 0 || (reinterpret_cast<uintptr_t>(a.Z) & 1) != 0) return false;
   const int64_t lim = int64_t(1) << 31;
   return a.M >= kI8aGemmMinM && a.M * a.N >= (kI8aGemmMinMacs + a.K - 1) / a.K && a.N * (a.K / 2) < lim && a.M * a.K < lim && (a.M + 31) / 32 * ((a.N + 31) / 32) < lim;
 }
