@@ -68,9 +68,51 @@ def test_qkv_mlp(both, M, dt, zp, skip, res):
     a, b, c = (q(g, n, K, bs, 4, zp, dt) for n in (N, Nkv, Nkv))
     both(lambda: ops.matmul_nbits_qkv(A, a[0], a[1], b[0], b[1], c[0], c[1], norm_scale=gm, skip=sk, block_size=bs,
                                       q_zero_points=a[2], k_zero_points=b[2], v_zero_points=c[2], want_residual=res))
+    both(lambda: ops.matmul_nbits_qkv(A, a[0], a[1], b[0], b[1], c[0], c[1], norm_scale=gm, block_size=bs, epsilon=1,
+                                      q_zero_points=a[2], k_zero_points=b[2], v_zero_points=c[2]))
     u = q(g, N, K, bs, 4, zp, dt)
     both(lambda: ops.matmul_nbits_mlp(A, a[0], a[1], u[0], u[1], skip=sk, norm_scale=gm if skip else None, block_size=bs,
                                       activation="gelu", gate_zero_points=a[2], up_zero_points=u[2], want_residual=res))
+
+
+@pytest.mark.parametrize("M,K,N,bits,dt", [(17, 512, 256, 4, torch.float32), (20, 256, 96, 8, torch.float16),
+                                           (128, 2048, 256, 4, torch.float16)])
+def test_workspace_call(both, M, K, N, bits, dt):
+    """A call that runs on a workspace comes back from the front end checked, as its bytes."""
+    from xrgpu_amd import ops
+    g = torch.Generator("cuda").manual_seed(M)
+    A = torch.randn(M, K, device="cuda", generator=g).to(dt)
+    B, S, Z = q(g, N, K, 32, bits, "packed", dt)
+    need = ops.matmul_nbits_workspace_bytes(M, K, N, bits, 32, dt)
+    assert need > 0 and ops._front().matmul(A, B, S, Z, None, None, None, bits, 32) == need
+    assert ops._front().matmul(A, B, S, Z[:, :-1], None, None, None, bits, 32) is None
+    both(lambda: ops.matmul_nbits(A, B, S, Z, bits=bits))
+
+
+def test_streams_and_threads(gpu):
+    """Each thread's calls run on its own stream, after the work enqueued there."""
+    from concurrent.futures import ThreadPoolExecutor
+    from xrgpu_amd import ops
+    g = torch.Generator("cuda").manual_seed(4)
+    B, S, Z = q(g, 96, 512, 32, 4, "packed", torch.float16)
+    As = [torch.randn(m, 512, device="cuda", generator=g).half() for m in (2, 70, 3, 130)]
+    want = [ops.matmul_nbits(2 * a, B, S, Z) for a in As]
+    torch.cuda.synchronize()
+
+    def work(a):
+        with torch.cuda.stream(torch.cuda.Stream()):
+            ys = []
+            for _ in range(8):
+                x = torch.zeros_like(a)
+                for _ in range(2):
+                    x += a
+                ys.append(ops.matmul_nbits(x, B, S, Z))
+            torch.cuda.current_stream().synchronize()
+            return ys
+
+    with ThreadPoolExecutor(4) as pool:
+        for ys, w in zip(pool.map(work, As), want):
+            assert all(torch.equal(y, w) for y in ys)
 
 
 def test_bnb4_gather(both):
@@ -86,6 +128,7 @@ def test_bnb4_gather(both):
     for dt in (torch.int32, torch.int64):
         idx = torch.tensor([3, 49, 0], dtype=dt, device="cuda")
         both(lambda: ops.gather_block_quantized(D, idx, S, bits=4, block_size=32, status=st, check=False))
+        both(lambda: ops.gather_block_quantized(D, idx, S, bits=4, block_size=32, status=st.view(torch.uint32), check=False))
 
 
 def test_declines(gpu):

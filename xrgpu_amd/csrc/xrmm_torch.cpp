@@ -6,7 +6,12 @@
 // Every function returns None, having done nothing, for whatever it does not take: a
 // tensor that is not a plain torch.Tensor on one GPU (subclasses, wrappers, CPU), any
 // mode that intercepts calls, a dtype, shape or layout that does not match, an empty
-// batch. ops.py then runs its own checks, which raise or accept as they always did.
+// batch. ops.py then runs its own checks, which raise or accept as they always did. A
+// MatMulNBits call that runs on a workspace comes back checked, as the workspace's
+// bytes (an int): ops.py, which keeps one per stream, makes the call. Declines are
+// return values and no exceptions: a throw costs 4 us, more than the checks (a float32
+// call on a workspace 17 x 1024 x 1024 took 18.7 us on the host with throws and every
+// check made twice, 15.8 without a front end).
 // Nothing is kept between calls. Measured, among other passes: Qkv 4 x 4096 x (4096 + 2 x
 // 1024) 17.8 -> 7.6 us a call, MatMulNBits 1 x 4096 x 14336 8.4 -> 6.9.
 #include <Python.h>
@@ -48,141 +53,143 @@ BnbFn g_bnb;
 GatherFn g_gather;
 PyObject *g_stream, *g_check;
 
-struct Decline {};  // ops.py takes the call
+// Helpers return false where ops.py takes the call.
 
-// a plain tensor on one GPU, contiguous; `dev` is the call's device (-1: not known yet)
-const at::Tensor& plain(PyObject* o, int& dev) {
-  if (!THPVariable_CheckExact(o)) throw Decline{};
+// A plain tensor on one GPU, contiguous; `dev` is the call's device (-1: not known yet).
+bool plain(PyObject* o, int& dev, const at::Tensor*& out) {
+  if (!THPVariable_CheckExact(o)) return false;
   const at::Tensor& t = THPVariable_Unpack(o);
   const auto ks = t.key_set();
   if (!t.is_cuda() || t.layout() != at::kStrided || ks.has(c10::DispatchKey::Python) ||
       ks.has_any(c10::functorch_transforms_ks) || t.is_conj() || t.is_neg() || !t.is_contiguous() || t.numel() == 0)
-    throw Decline{};
+    return false;
   const int d = t.get_device();
   if (dev < 0) dev = d;
-  if (d != dev) throw Decline{};
-  return t;
+  out = &t;
+  return d == dev;
 }
 
 bool none(PyObject* o) { return o == Py_None; }
 
-int64_t integer(PyObject* o) {
-  if (!PyLong_CheckExact(o)) throw Decline{};
-  const int64_t v = PyLong_AsLongLong(o);
-  if (v == -1 && PyErr_Occurred()) {
-    PyErr_Clear();
-    throw Decline{};
+bool integer(PyObject* o, int64_t& v) {
+  if (!PyLong_CheckExact(o)) return false;
+  int over = 0;
+  v = PyLong_AsLongLongAndOverflow(o, &over);
+  return over == 0;
+}
+
+bool real(PyObject* o, float& v) {
+  if (PyFloat_CheckExact(o)) {
+    v = static_cast<float>(PyFloat_AS_DOUBLE(o));
+    return true;
   }
-  return v;
+  int64_t i = 0;
+  if (!integer(o, i)) return false;
+  v = static_cast<float>(static_cast<double>(i));
+  return true;
 }
 
-double real(PyObject* o) {
-  if (!PyFloat_CheckExact(o)) throw Decline{};
-  return PyFloat_AS_DOUBLE(o);
-}
-
-void want(bool ok) {
-  if (!ok) throw Decline{};
+// None or the integer n
+bool none_or(PyObject* o, int64_t n) {
+  int64_t v = 0;
+  return none(o) || (integer(o, v) && v == n);
 }
 
 bool shape(const at::Tensor& t, std::initializer_list<int64_t> s) { return t.sizes() == at::IntArrayRef(s.begin(), s.size()); }
 
-int t1(const at::Tensor& a) {
-  if (a.scalar_type() == at::kHalf) return F16;
-  want(a.scalar_type() == at::kFloat);
-  return F32;
+bool t1(const at::Tensor& a, int& dt) {
+  dt = a.scalar_type() == at::kHalf ? F16 : F32;
+  return dt == F16 || a.scalar_type() == at::kFloat;
 }
 
-void* stream_of(int dev) {
+bool stream_of(int dev, void*& s) {
   PyObject* i = PyLong_FromLong(dev);
   PyObject* r = i ? PyObject_CallOneArg(g_stream, i) : nullptr;
   Py_XDECREF(i);
-  if (!r) {
-    PyErr_Clear();
-    throw Decline{};
-  }
-  void* s = PyLong_AsVoidPtr(r);
-  Py_DECREF(r);
+  s = r ? PyLong_AsVoidPtr(r) : nullptr;
+  Py_XDECREF(r);
   if (s == nullptr && PyErr_Occurred()) {
     PyErr_Clear();
-    throw Decline{};
+    return false;
   }
-  return s;
+  return true;
 }
 
 // rows, K and the leading axes of the activations
 struct Act {
-  const at::Tensor& A;
-  int64_t K, M;
-  int dt;
-  at::DimVector lead;
-  Act(const at::Tensor& a, PyObject* k) : A(a), K(0), M(0), dt(t1(a)) {
-    want(a.dim() >= 1);
-    K = a.size(-1);
-    want(none(k) || integer(k) == K);
-    M = a.numel() / K;
-    lead = at::DimVector(a.sizes().slice(0, a.dim() - 1));
+  const at::Tensor* A = nullptr;
+  int64_t K = 0, M = 0;
+  int dt = F32;
+  bool set(PyObject* a, PyObject* k, int& dev) {
+    if (!plain(a, dev, A) || !t1(*A, dt) || A->dim() < 1) return false;
+    K = A->size(-1);
+    M = A->numel() / K;
+    return none_or(k, K);
   }
+  const void* data() const { return A->data_ptr(); }
   at::Tensor out(int64_t n) const {
-    at::DimVector s = lead;
+    at::DimVector s(A->sizes().slice(0, A->dim() - 1));
     s.push_back(n);
-    return at::empty(s, A.options());
+    return at::empty(s, A->options());
   }
 };
 
 struct Quant {
-  int bits, bs;
-  int64_t kb, blob, zrow;
-  Quant(PyObject* b, PyObject* s, int64_t K) {
-    const int64_t bb = integer(b), ss = integer(s);
-    want((bb == 2 || bb == 4 || bb == 8) && ss > 0 && ss <= (1 << 20));
+  int bits = 0, bs = 0;
+  int64_t kb = 0, blob = 0, zrow = 0;
+  bool set(PyObject* b, PyObject* s, int64_t K) {
+    int64_t bb = 0, ss = 0;
+    if (!integer(b, bb) || !integer(s, ss) || !(bb == 2 || bb == 4 || bb == 8) || ss <= 0 || ss > (1 << 20)) return false;
     bits = static_cast<int>(bb);
     bs = static_cast<int>(ss);
     kb = (K + bs - 1) / bs;
     blob = (static_cast<int64_t>(bs) * bits + 7) / 8;
     zrow = (kb * bits + 7) / 8;
+    return true;
   }
 };
 
 struct Weights {
-  const void *B, *S, *Z;
-  int zdt;
-  int64_t N;
+  const void *B = nullptr, *S = nullptr, *Z = nullptr;
+  int zdt = UNSPECIFIED;
+  int64_t N = 0;
+  bool set(PyObject* b, PyObject* s, PyObject* z, PyObject* n, const Act& a, const Quant& q, int& dev) {
+    const at::Tensor *tb, *ts, *tz;
+    if (!plain(b, dev, tb) || !plain(s, dev, ts) || tb->scalar_type() != at::kByte || tb->dim() != 3) return false;
+    N = tb->size(0);
+    if (!none_or(n, N) || !shape(*tb, {N, q.kb, q.blob}) || ts->scalar_type() != a.A->scalar_type() || !shape(*ts, {N, q.kb}))
+      return false;
+    B = tb->data_ptr();
+    S = ts->data_ptr();
+    if (none(z)) return true;
+    if (!plain(z, dev, tz)) return false;
+    const bool packed = tz->scalar_type() == at::kByte;
+    if (packed) zdt = U8;
+    else if (!t1(*tz, zdt)) return false;
+    Z = tz->data_ptr();
+    return shape(*tz, {N, packed ? q.zrow : q.kb});
+  }
 };
 
-Weights weights(PyObject* b, PyObject* s, PyObject* z, PyObject* n, const Act& a, const Quant& q, int& dev) {
-  const at::Tensor &B = plain(b, dev), &S = plain(s, dev);
-  want(B.scalar_type() == at::kByte && B.dim() == 3);
-  const int64_t N = B.size(0);
-  want((none(n) || integer(n) == N) && shape(B, {N, q.kb, q.blob}) && S.scalar_type() == a.A.scalar_type() && shape(S, {N, q.kb}));
-  Weights w{B.data_ptr(), S.data_ptr(), nullptr, UNSPECIFIED, N};
-  if (!none(z)) {
-    const at::Tensor& Z = plain(z, dev);
-    const bool packed = Z.scalar_type() == at::kByte;
-    w.zdt = packed ? U8 : t1(Z);
-    want(shape(Z, {N, packed ? q.zrow : q.kb}));
-    w.Z = Z.data_ptr();
-  }
-  return w;
-}
-
 // an optional tensor of A's dtype with n elements (vec: one-dimensional)
-const void* aux(PyObject* o, const Act& a, int64_t n, bool vec, int& dev) {
-  if (none(o)) return nullptr;
-  const at::Tensor& t = plain(o, dev);
-  want(t.scalar_type() == a.A.scalar_type() && t.numel() == n && (!vec || t.dim() == 1));
-  return t.data_ptr();
+bool aux(PyObject* o, const Act& a, int64_t n, bool vec, int& dev, const void*& p) {
+  p = nullptr;
+  if (none(o)) return true;
+  const at::Tensor* t;
+  if (!plain(o, dev, t) || t->scalar_type() != a.A->scalar_type() || t->numel() != n || (vec && t->dim() != 1)) return false;
+  p = t->data_ptr();
+  return true;
 }
 
 // the projections' common zero-point dtype
-int one_zdt(std::initializer_list<const Weights*> ws) {
-  int dt = UNSPECIFIED;
+bool one_zdt(std::initializer_list<const Weights*> ws, int& dt) {
+  dt = UNSPECIFIED;
   for (const Weights* w : ws)
     if (w->Z) {
-      want(dt == UNSPECIFIED || dt == w->zdt);
+      if (dt != UNSPECIFIED && dt != w->zdt) return false;
       dt = w->zdt;
     }
-  return dt;
+  return true;
 }
 
 bool checked(int rc) {  // false: the Python error is set
@@ -210,30 +217,35 @@ PyObject* guarded(Py_ssize_t n, Py_ssize_t expected, F&& f) {
   if (n != expected || c10::impl::dispatch_mode_enabled() || at::impl::torch_function_mode_enabled()) Py_RETURN_NONE;
   try {
     return f();
-  } catch (const Decline&) {
-    Py_RETURN_NONE;
   } catch (const std::exception& e) {  // an allocation that failed, say: ops.py meets it again
     Py_RETURN_NONE;
   }
 }
 
-// (A, B, scales, zero_points, bias, K, N, bits, block_size)
+// (A, B, scales, zero_points, bias, K, N, bits, block_size); an int: checked, needs a
+// workspace of that many bytes
 PyObject* matmul(PyObject*, PyObject* const* v, Py_ssize_t n) {
   return guarded(n, 9, [&]() -> PyObject* {
     int dev = -1;
-    const Act a(plain(v[0], dev), v[5]);
-    const Quant q(v[7], v[8], a.K);
-    const Weights w = weights(v[1], v[2], v[3], v[6], a, q, dev);
-    const void* bias = aux(v[4], a, w.N, true, dev);
-    // calls on a workspace stay with ops.py, which keeps one per stream
-    if (a.M > 4 && g_matmul_ws(a.M, a.K, w.N, q.bits, q.bs, a.dt) > 0) throw Decline{};
-    void* st = stream_of(dev);
+    Act a;
+    Quant q;
+    Weights w;
+    const void* bias;
+    if (!a.set(v[0], v[5], dev) || !q.set(v[7], v[8], a.K) || !w.set(v[1], v[2], v[3], v[6], a, q, dev) ||
+        !aux(v[4], a, w.N, true, dev, bias))
+      Py_RETURN_NONE;
+    if (a.M > 4) {
+      const int64_t need = g_matmul_ws(a.M, a.K, w.N, q.bits, q.bs, a.dt);
+      if (need > 0) return PyLong_FromLongLong(need);
+    }
+    void* st;
+    if (!stream_of(dev, st)) Py_RETURN_NONE;
     at::Tensor y;
     int rc;
     {
       NoGil ng;
       y = a.out(w.N);
-      rc = g_matmul(a.A.data_ptr(), w.B, w.S, w.Z, w.zdt, bias, y.data_ptr(), a.M, a.K, w.N, q.bits, q.bs, a.dt, st);
+      rc = g_matmul(a.data(), w.B, w.S, w.Z, w.zdt, bias, y.data_ptr(), a.M, a.K, w.N, q.bits, q.bs, a.dt, st);
     }
     if (!checked(rc)) return nullptr;
     return THPVariable_Wrap(y);
@@ -246,26 +258,25 @@ at::Tensor scratch(int op, const Act& a, int64_t N, int64_t Nkv, const Quant& q,
     bytes = 0;
     return {};
   }
-  return at::empty({bytes}, a.A.options().dtype(at::kByte));
+  return at::empty({bytes}, a.A->options().dtype(at::kByte));
 }
 
 // (A, q_B, q_scales, k_B, k_scales, v_B, v_scales, norm_scale, skip, K, Nq, Nkv, bits,
 //  block_size, epsilon, q_zero_points, k_zero_points, v_zero_points, want_residual)
 PyObject* qkv(PyObject*, PyObject* const* v, Py_ssize_t n) {
   return guarded(n, 19, [&]() -> PyObject* {
-    int dev = -1;
-    const Act a(plain(v[0], dev), v[9]);
-    const Quant q(v[12], v[13], a.K);
-    const Weights wq = weights(v[1], v[2], v[15], v[10], a, q, dev);
-    const Weights wk = weights(v[3], v[4], v[16], v[11], a, q, dev);
-    const Weights wv = weights(v[5], v[6], v[17], v[11], a, q, dev);
-    want(wk.N == wv.N && !none(v[7]));
-    const int zdt = one_zdt({&wq, &wk, &wv});
-    const void* gamma = aux(v[7], a, a.K, true, dev);
-    const void* skip = aux(v[8], a, a.M * a.K, false, dev);
-    const float eps = static_cast<float>(real(v[14]));
-    want(PyBool_Check(v[18]));
-    void* st = stream_of(dev);
+    int dev = -1, zdt;
+    Act a;
+    Quant q;
+    Weights wq, wk, wv;
+    const void *gamma, *skip;
+    void* st;
+    float eps;
+    if (!real(v[14], eps) || !PyBool_Check(v[18]) || none(v[7]) || !a.set(v[0], v[9], dev) || !q.set(v[12], v[13], a.K) || !wq.set(v[1], v[2], v[15], v[10], a, q, dev) ||
+        !wk.set(v[3], v[4], v[16], v[11], a, q, dev) || !wv.set(v[5], v[6], v[17], v[11], a, q, dev) || wk.N != wv.N ||
+        !one_zdt({&wq, &wk, &wv}, zdt) || !aux(v[7], a, a.K, true, dev, gamma) ||
+        !aux(v[8], a, a.M * a.K, false, dev, skip) || !stream_of(dev, st))
+      Py_RETURN_NONE;
     const bool residual = v[18] == Py_True;
     at::Tensor Q, Ko, V, R;
     int rc;
@@ -275,7 +286,7 @@ PyObject* qkv(PyObject*, PyObject* const* v, Py_ssize_t n) {
       if (residual) R = a.out(a.K);
       int64_t nws = 0;
       const at::Tensor ws = scratch(1, a, wq.N, wk.N, q, skip != nullptr, true, nws);
-      rc = g_qkv(a.A.data_ptr(), skip, gamma, wq.B, wq.S, wq.Z, wk.B, wk.S, wk.Z, wv.B, wv.S, wv.Z, zdt, Q.data_ptr(),
+      rc = g_qkv(a.data(), skip, gamma, wq.B, wq.S, wq.Z, wk.B, wk.S, wk.Z, wv.B, wv.S, wv.Z, zdt, Q.data_ptr(),
                  Ko.data_ptr(), V.data_ptr(), residual ? R.data_ptr() : nullptr, a.M, a.K, wq.N, wk.N, q.bits, q.bs, eps, a.dt,
                  nws ? ws.data_ptr() : nullptr, nws, st);
     }
@@ -289,19 +300,19 @@ PyObject* qkv(PyObject*, PyObject* const* v, Py_ssize_t n) {
 //  block_size, epsilon, activation code, gate_zero_points, up_zero_points, want_residual)
 PyObject* mlp(PyObject*, PyObject* const* v, Py_ssize_t n) {
   return guarded(n, 18, [&]() -> PyObject* {
-    int dev = -1;
-    const Act a(plain(v[0], dev), v[9]);
-    const Quant q(v[11], v[12], a.K);
-    const Weights g = weights(v[1], v[2], v[15], v[10], a, q, dev), u = weights(v[3], v[4], v[16], v[10], a, q, dev);
-    want(g.N == u.N);
-    const int zdt = one_zdt({&g, &u});
-    const void* skip = aux(v[5], a, a.M * a.K, false, dev);
-    const void* gamma = aux(v[6], a, a.K, true, dev);
-    const void *gb = aux(v[7], a, g.N, true, dev), *ub = aux(v[8], a, g.N, true, dev);
-    const float eps = static_cast<float>(real(v[13]));
-    const int act = static_cast<int>(integer(v[14]));
-    want(PyBool_Check(v[17]));
-    void* st = stream_of(dev);
+    int dev = -1, zdt;
+    Act a;
+    Quant q;
+    Weights g, u;
+    const void *skip, *gamma, *gb, *ub;
+    int64_t act = 0;
+    void* st;
+    float eps;
+    if (!real(v[13], eps) || !integer(v[14], act) || !PyBool_Check(v[17]) || !a.set(v[0], v[9], dev) || !q.set(v[11], v[12], a.K) || !g.set(v[1], v[2], v[15], v[10], a, q, dev) ||
+        !u.set(v[3], v[4], v[16], v[10], a, q, dev) || g.N != u.N || !one_zdt({&g, &u}, zdt) ||
+        !aux(v[5], a, a.M * a.K, false, dev, skip) || !aux(v[6], a, a.K, true, dev, gamma) || !aux(v[7], a, g.N, true, dev, gb) ||
+        !aux(v[8], a, g.N, true, dev, ub) || !stream_of(dev, st))
+      Py_RETURN_NONE;
     const bool residual = v[17] == Py_True;
     at::Tensor Y, R;
     int rc;
@@ -311,8 +322,8 @@ PyObject* mlp(PyObject*, PyObject* const* v, Py_ssize_t n) {
       if (residual) R = a.out(a.K);
       int64_t nws = 0;
       const at::Tensor ws = scratch(2, a, g.N, 0, q, skip != nullptr, gamma != nullptr, nws);
-      rc = g_mlp(a.A.data_ptr(), skip, gamma, g.B, g.S, g.Z, gb, u.B, u.S, u.Z, ub, zdt, Y.data_ptr(),
-                 residual ? R.data_ptr() : nullptr, a.M, a.K, g.N, q.bits, q.bs, eps, act, a.dt,
+      rc = g_mlp(a.data(), skip, gamma, g.B, g.S, g.Z, gb, u.B, u.S, u.Z, ub, zdt, Y.data_ptr(),
+                 residual ? R.data_ptr() : nullptr, a.M, a.K, g.N, q.bits, q.bs, eps, static_cast<int>(act), a.dt,
                  nws ? ws.data_ptr() : nullptr, nws, st);
     }
     if (!checked(rc)) return nullptr;
@@ -325,19 +336,24 @@ PyObject* mlp(PyObject*, PyObject* const* v, Py_ssize_t n) {
 PyObject* bnb4(PyObject*, PyObject* const* v, Py_ssize_t n) {
   return guarded(n, 8, [&]() -> PyObject* {
     int dev = -1;
-    const Act a(plain(v[0], dev), v[3]);
-    const at::Tensor &B = plain(v[1], dev), &S = plain(v[2], dev);
-    const int64_t N = integer(v[4]), bs = integer(v[5]), qt = integer(v[6]), tb = integer(v[7]);
-    want(a.A.dim() == 2 && N > 0 && N < (int64_t(1) << 31) && a.K < (int64_t(1) << 31) && bs > 0 && bs <= (1 << 20) && B.scalar_type() == at::kByte &&
-         S.scalar_type() == a.A.scalar_type() && B.numel() >= (N * a.K + 1) / 2 && S.numel() >= (N * a.K + bs - 1) / bs &&
-         (qt == 0 || qt == 1) && (tb == 0 || tb == 1));
-    void* st = stream_of(dev);
+    Act a;
+    const at::Tensor *B, *S;
+    int64_t N = 0, bs = 0, qt = 0, tb = 0;
+    void* st;
+    if (!a.set(v[0], v[3], dev) || !plain(v[1], dev, B) || !plain(v[2], dev, S) || !integer(v[4], N) || !integer(v[5], bs) ||
+        !integer(v[6], qt) || !integer(v[7], tb))
+      Py_RETURN_NONE;
+    const int64_t lim = int64_t(1) << 31;
+    if (a.A->dim() != 2 || N <= 0 || N >= lim || a.K >= lim || bs <= 0 || bs > (1 << 20) || B->scalar_type() != at::kByte ||
+        S->scalar_type() != a.A->scalar_type() || B->numel() < (N * a.K + 1) / 2 || S->numel() < (N * a.K + bs - 1) / bs ||
+        !(qt == 0 || qt == 1) || !(tb == 0 || tb == 1) || !stream_of(dev, st))
+      Py_RETURN_NONE;
     at::Tensor y;
     int rc;
     {
       NoGil ng;
       y = a.out(N);
-      rc = g_bnb(a.A.data_ptr(), B.data_ptr(), S.data_ptr(), y.data_ptr(), a.M, a.K, N, static_cast<int32_t>(bs),
+      rc = g_bnb(a.data(), B->data_ptr(), S->data_ptr(), y.data_ptr(), a.M, a.K, N, static_cast<int32_t>(bs),
                  static_cast<int32_t>(qt), static_cast<int32_t>(tb), a.dt, st);
     }
     if (!checked(rc)) return nullptr;
@@ -349,28 +365,30 @@ PyObject* bnb4(PyObject*, PyObject* const* v, Py_ssize_t n) {
 PyObject* gather(PyObject*, PyObject* const* v, Py_ssize_t n) {
   return guarded(n, 7, [&]() -> PyObject* {
     int dev = -1;
-    const at::Tensor &D = plain(v[0], dev), &I = plain(v[1], dev), &S = plain(v[2], dev), &st_t = plain(v[4], dev);
-    const int64_t bits = integer(v[5]), bs = integer(v[6]);
-    want((bits == 4 || bits == 8) && bs > 0 && bs <= (1 << 20) && D.scalar_type() == at::kByte && D.dim() == 2 && I.dim() == 1 &&
-         S.scalar_type() == at::kFloat && st_t.scalar_type() == at::kInt);
-    const bool i64 = I.scalar_type() == at::kLong;
-    want(i64 || I.scalar_type() == at::kInt);
-    const int64_t rows = D.size(0), pcols = D.size(1), width = pcols * (8 / bits), blocks = (width + bs - 1) / bs;
-    want(shape(S, {rows, blocks}));
+    const at::Tensor *D, *I, *S, *T, *Z;
+    int64_t bits = 0, bs = 0;
+    if (!plain(v[0], dev, D) || !plain(v[1], dev, I) || !plain(v[2], dev, S) || !plain(v[4], dev, T) || !integer(v[5], bits) ||
+        !integer(v[6], bs) || !(bits == 4 || bits == 8) || bs <= 0 || bs > (1 << 20) || D->scalar_type() != at::kByte ||
+        D->dim() != 2 || I->dim() != 1 || S->scalar_type() != at::kFloat ||
+        !(T->scalar_type() == at::kInt || T->scalar_type() == at::kUInt32))
+      Py_RETURN_NONE;
+    const bool i64 = I->scalar_type() == at::kLong;
+    const int64_t rows = D->size(0), pcols = D->size(1), width = pcols * (8 / bits), blocks = (width + bs - 1) / bs;
+    if (!(i64 || I->scalar_type() == at::kInt) || !shape(*S, {rows, blocks})) Py_RETURN_NONE;
     const void* z = nullptr;
     if (!none(v[3])) {
-      const at::Tensor& Z = plain(v[3], dev);
-      want(Z.scalar_type() == at::kByte && shape(Z, {rows, (blocks * bits + 7) / 8}));
-      z = Z.data_ptr();
+      if (!plain(v[3], dev, Z) || Z->scalar_type() != at::kByte || !shape(*Z, {rows, (blocks * bits + 7) / 8})) Py_RETURN_NONE;
+      z = Z->data_ptr();
     }
-    void* st = stream_of(dev);
+    void* st;
+    if (!stream_of(dev, st)) Py_RETURN_NONE;
     at::Tensor y;
     int rc;
     {
       NoGil ng;
-      y = at::empty({I.size(0), width}, S.options());
-      rc = g_gather(D.data_ptr(), I.data_ptr(), i64 ? 7 : 2, S.data_ptr(), z, y.data_ptr(), st_t.data_ptr(), rows, pcols,
-                    I.size(0), static_cast<int32_t>(bits), static_cast<int32_t>(bs), st);
+      y = at::empty({I->size(0), width}, S->options());
+      rc = g_gather(D->data_ptr(), I->data_ptr(), i64 ? 7 : 2, S->data_ptr(), z, y.data_ptr(), T->data_ptr(), rows, pcols,
+                    I->size(0), static_cast<int32_t>(bits), static_cast<int32_t>(bs), st);
     }
     if (!checked(rc)) return nullptr;
     return THPVariable_Wrap(y);

@@ -42,8 +42,8 @@ def _stream(stream=None, device=None):
 
 
 # The native front end (csrc/xrmm_torch.cpp): None until first asked for, False where it
-# is not built, built for another torch, or there is no GPU. Its functions return None for whatever they do not
-# take, and the checks below then decide.
+# is not built, built for another torch, or there is no GPU. Its functions return None
+# for whatever they do not take, and the checks below then decide.
 _FRONT = None
 
 
@@ -169,25 +169,29 @@ def matmul_nbits(A, B, scales, zero_points=None, bias=None, *, K=None, N=None, b
     need different workspaces. Under HIP graph capture without a caller
     workspace the call runs unsplit, so a captured graph never depends on a
     workspace this module might replace or share with another graph."""
+    need = None
     if out is None and workspace is None and stream is None and _front():
-        y = _FRONT.matmul(A, B, scales, zero_points, bias, K, N, bits, block_size)
-        if y is not None:
-            return y
+        need = _FRONT.matmul(A, B, scales, zero_points, bias, K, N, bits, block_size)
+        if need is not None and type(need) is not int:
+            return need
     K = int(K if K is not None else A.shape[-1])
     N = int(N if N is not None else B.shape[0])
-    if A.shape[-1] != K:
-        raise nat.XrmmInvalid("A's last dimension must equal K")
-    _check_weights(B, scales, zero_points, N, K, bits, block_size, A.dtype)
-    if bias is not None and (bias.dtype != A.dtype or tuple(bias.shape) != (N,)):
-        raise nat.XrmmInvalid("bias must be [N] of A's dtype")
-    M = A.numel() // K
-    _check_out(out, tuple(A.shape[:-1]) + (N,), A.dtype)
-    dev = _check_dev(A, B, scales, zero_points, bias, out)
+    if need is None:
+        if A.shape[-1] != K:
+            raise nat.XrmmInvalid("A's last dimension must equal K")
+        _check_weights(B, scales, zero_points, N, K, bits, block_size, A.dtype)
+        if bias is not None and (bias.dtype != A.dtype or tuple(bias.shape) != (N,)):
+            raise nat.XrmmInvalid("bias must be [N] of A's dtype")
+        M = A.numel() // K
+        _check_out(out, tuple(A.shape[:-1]) + (N,), A.dtype)
+        dev = _check_dev(A, B, scales, zero_points, bias, out)
+        lib = nat.lib()
+        need = lib.xrmm_matmul_nbits_workspace_bytes(M, K, N, bits, block_size, _t1(A)) if M > 4 else 0
+    else:  # an int: the front end has checked the call, which needs a workspace of that many bytes
+        M, dev, lib = A.numel() // K, A.get_device(), nat.lib()
     if out is None:
         out = torch.empty(tuple(A.shape[:-1]) + (N,), dtype=A.dtype, device=A.device)
-    lib = nat.lib()
     s = _stream(stream, dev)
-    need = lib.xrmm_matmul_nbits_workspace_bytes(M, K, N, bits, block_size, _t1(A)) if M > 4 else 0
     if need > 0 and workspace is not None:
         if workspace.dtype != torch.uint8 or workspace.numel() < need or workspace.get_device() != dev:
             raise nat.XrmmInvalid(f"workspace must be uint8 with at least {need} bytes on A's device")
