@@ -281,3 +281,68 @@ def test_grouped_tiny_rows(gpu, act, scale, bs):
     assert np.all(got[9] == 0)
     ok, err, lim = O.tolerance_ok(got[3], ref[3], np.float32)
     assert ok and np.isfinite(got[3]).all() and np.abs(ref[3]).max() > 0, (err, lim)
+
+
+def tile_rows(pairs, E, cols, bits, bs):
+    """The dispatch's rule on 256 CUs: pairs per row tile of a GEMM with `cols` column tiles."""
+    alone, both, half = (0.8, 1.3, 0.75) if bs else (0.6, 1.0, 0.7)
+    quarter = 1.0 if not bs else 0.9 if bits == 4 else 0.6
+    p = pairs / E
+
+    def tiles(rt):
+        return min(E, pairs) * (np.ceil(p / rt) + np.ceil((p + 1.3 * p ** 0.5) / rt)) / 2 * cols
+    full, rest = divmod(tiles(64) / 512, 1)
+    c64 = full * both + (0 if rest == 0 else alone if rest <= 0.5 else both)
+    c128 = np.ceil(tiles(128) / 256) * (quarter if p <= 32 else half if p <= 64 else 1.0)
+    return 64 if c64 <= c128 + 1e-9 else 128
+
+
+TILES = [  # H, I, activation, bits, block, FC1's and FC2's pairs per tile
+    (192, 7680, "relu", 4, 64, 64, 128),     # three steps: a super-step of one
+    (128, 7680, "relu", 4, 32, 64, 128),
+    (7680, 128, "relu", 4, 64, 128, 64),
+    (7680, 128, "relu", 8, 128, 128, 64),
+    (128, 3840, "swiglu", 8, 64, 64, 128),
+    (192, 3840, "swiglu", 8, 32, 64, 128),
+    (128, 3840, "swiglu", 4, 128, 64, 128),
+    (7680, 256, "relu", 4, 256, 128, 64),    # blocks longer than a super-step
+    (256, 7680, "relu", 8, 256, 64, 128),
+    (192, 3840, "swiglu", 4, 0, 64, 64),
+    (192, 7168, "relu", 8, 0, 128, 64),
+    (256, 256, "swiglu", 8, 32, 128, 128),
+]
+
+
+@pytest.mark.parametrize("H,I,act,bits,bs,r1,r2", TILES)
+def test_grouped_tile_heights(gpu, H, I, act, bits, bs, r1, r2):
+    """Both tile heights in both GEMMs, with experts of no pair, one, and one less and one
+    more than whole tiles; every expert's first, last and a middle token against the oracle."""
+    if torch.cuda.get_device_properties(0).multi_processor_count != 256:
+        pytest.skip("the expected heights are those of 256 CUs")
+    counts = [1, 64, 65, 32, 33, 129, 0, 96, 102]
+    T, E, sw = sum(counts), len(counts), act == "swiglu"
+    rng = np.random.default_rng(H + I + bits + bs)
+    i = rand_case(rng, T, H, I, E, bits, bs, sw)
+    F1 = i["fc1T"].shape[1]
+    ks = max(1, min(-(-512 // (-(-T // 64) * -(-H // 256))), 4, I // 1024))
+    assert (tile_rows(T, E, -(-F1 // 256), bits, bs), tile_rows(T, E, -(-H // 256) * ks, bits, bs)) == (r1, r2)
+    expert = rng.permutation(np.repeat(np.arange(E), counts))
+    i["routerT"] = (rng.standard_normal((T, E)) * 0.1 + 8.0 * (np.arange(E) == expert[:, None])).astype(np.float32)
+    at = dict(k=1, activation=act, swiglu_fusion=1 if sw else 0, bits=bits, block_size=bs, alpha=1.0, beta=0.0,
+              swiglu_limit=None)
+    assert ops().qmoe_kernel(T, H, E, F1, 1, bits, bs, act, 1 if sw else 0) == "qmoe_grouped"
+    got = run_gpu(i, at)
+    pick = sorted({t for e in range(E) if counts[e] for t in np.flatnonzero(expert == e)[[0, counts[e] // 2, -1]]})
+    ref = run_oracle(dict(i, inputT=i["inputT"][pick], routerT=i["routerT"][pick]), at)
+    ok, err, lim = O.tolerance_ok(got[pick], ref, np.float32)
+    assert ok and np.isfinite(got).all(), (err, lim)
+
+
+def test_grouped_many_experts(gpu):
+    """More experts than the workspace has separate row-tile offsets for: both GEMMs share one height."""
+    T, H, I, E = 40, 64, 64, 2800
+    i = rand_case(np.random.default_rng(5), T, H, I, E, 4, 32, False)
+    at = dict(k=2, activation="relu", swiglu_fusion=0, bits=4, block_size=32, alpha=1.0, beta=0.0, swiglu_limit=None)
+    assert ops().qmoe_kernel(T, H, E, I, 2, 4, 32, "relu", 0) == "qmoe_grouped"
+    ok, err, lim = O.tolerance_ok(run_gpu(i, at), run_oracle(i, at), np.float32)
+    assert ok, (err, lim)

@@ -26,12 +26,15 @@
 // multiplies the sum of its block (or the row's total for row scales). Other
 // geometries take a routing kernel and one-thread-per-output kernels.
 #include <algorithm>
+#include <cmath>
 #include <type_traits>
 
 #include "xrmm_device.h"
 #include "xrmm_moe.h"
 
 namespace xrmm {
+
+int device_cus();
 
 namespace {
 
@@ -640,10 +643,10 @@ const char* moe_kernel_name(const MoeArgs& a) {
 
 namespace {
 // One grouped GEMM launch of stage ST, BITS-bit codes, block mode BKM.
-template <int ST, int BITS, int BKM>
+template <int ST, int BITS, int BKM, int RT>
 hipError_t mg_launch(const MoeArgs& a, const MgLists& g, int nct, int64_t grid, hipStream_t st) {
-  auto kern = k_moe_ggemm<ST, BITS, BKM>;
-  constexpr size_t lds = mg_lds<BITS, BKM>();
+  auto kern = k_moe_ggemm<ST, BITS, BKM, RT>;
+  constexpr size_t lds = mg_lds<BITS, BKM, RT>();
   if constexpr (lds > 64 * 1024) {
     static std::atomic<int> done[kMaxDevices];  // per instantiation and device
     if (hipError_t e = raise_lds_cap(reinterpret_cast<const void*>(kern), static_cast<int>(lds), done); e != hipSuccess)
@@ -653,29 +656,64 @@ hipError_t mg_launch(const MoeArgs& a, const MgLists& g, int nct, int64_t grid, 
   return hipGetLastError();
 }
 
-template <int ST, int BITS>
+template <int ST, int BITS, int RT>
 hipError_t mg_launch_b(const MoeArgs& a, const MgLists& g, int nct, int64_t grid, hipStream_t st) {
   switch (mg_block_mode(a.bs)) {  // blocks of 16 (mode 1) do not take this path
-    case 0: return mg_launch<ST, BITS, 0>(a, g, nct, grid, st);
-    case 2: return mg_launch<ST, BITS, 2>(a, g, nct, grid, st);
-    case 4: return mg_launch<ST, BITS, 4>(a, g, nct, grid, st);
-    default: return mg_launch<ST, BITS, 8>(a, g, nct, grid, st);
+    case 0: return mg_launch<ST, BITS, 0, RT>(a, g, nct, grid, st);
+    case 2: return mg_launch<ST, BITS, 2, RT>(a, g, nct, grid, st);
+    case 4: return mg_launch<ST, BITS, 4, RT>(a, g, nct, grid, st);
+    default: return mg_launch<ST, BITS, 8, RT>(a, g, nct, grid, st);
   }
 }
 
 template <int ST>
-hipError_t mg_launch_s(const MoeArgs& a, const MgLists& g, int nct, int64_t grid, hipStream_t st) {
-  return a.bits == 8 ? mg_launch_b<ST, 8>(a, g, nct, grid, st) : mg_launch_b<ST, 4>(a, g, nct, grid, st);
+hipError_t mg_launch_s(const MoeArgs& a, const MgLists& g, int rt, int nct, int64_t grid, hipStream_t st) {
+  if (rt == 64) return a.bits == 8 ? mg_launch_b<ST, 8, 64>(a, g, nct, grid, st) : mg_launch_b<ST, 4, 64>(a, g, nct, grid, st);
+  return a.bits == 8 ? mg_launch_b<ST, 8, 128>(a, g, nct, grid, st) : mg_launch_b<ST, 4, 128>(a, g, nct, grid, st);
+}
+
+// Pairs per row tile (128 or 64) of a GEMM of the grouped path with `cols` column tiles
+// (times K splits): the cheaper by rounds of workgroups on the CUs, in units of a round
+// of full 128-pair tiles. One 128-pair workgroup fills a CU; its round costs `half` with
+// at most 64 pairs in a tile and `quarter` with at most 32. Two 64-pair workgroups share
+// a CU, a round of them costs `both`, a last round of single ones `alone`. The pairs of
+// an expert are taken as T k / E, and that plus 1.3 of its square root (routing is not
+// even), half and half.
+//
+// The four costs fit 785 sizes (T k from 32, H 1024 .. 4096, I 768 .. 14336, 8 .. 32
+// experts), each GEMM timed with both heights. Against 128-pair tiles alone: 9 % less
+// time in the mean (row scales 13 %: without scaled sums the second dequantisation is all
+// that 64-pair tiles add; 8-bit blocks 6 %: 64 bytes of a column are one step, so the
+// codes arrive late when few pairs leave a step short), 20 sizes 2 to 8 % more.
+int mg_tile_rows(const MoeArgs& a, int64_t cols) {
+  const double alone = a.bs ? 0.8 : 0.6, both = a.bs ? 1.3 : 1.0, half = a.bs ? 0.75 : 0.7,
+               quarter = a.bs == 0 ? 1.0 : a.bits == 4 ? 0.9 : 0.6;
+  const int n = device_cus();
+  const double cus = n > 0 ? n : 256, pairs = static_cast<double>(a.T * a.k), p = pairs / static_cast<double>(a.E);
+  auto tiles = [&](double rt) {
+    return std::min(static_cast<double>(a.E), pairs) * (std::ceil(p / rt) + std::ceil((p + 1.3 * std::sqrt(p)) / rt)) / 2 *
+           static_cast<double>(cols);
+  };
+  const double r64 = tiles(64) / (2 * cus), full = std::floor(r64), rest = r64 - full;
+  const double c64 = full * both + (rest == 0 ? 0.0 : rest <= 0.5 ? alone : both);
+  const double c128 = std::ceil(tiles(128) / cus) * (p <= 32 ? quarter : p <= 64 ? half : 1.0);
+  return c64 <= c128 + 1e-9 ? 64 : 128;
 }
 
 hipError_t launch_grouped(const MoeArgs& a0, hipStream_t st) {
   MoeArgs a = a0;
   a.ks = static_cast<int>(moe_group_fc2_splits(a.T, a.k, a.H, a.I));  // FC2 K splits (the combine sums them)
+  const int nct1 = static_cast<int>((a.F1 + MG_CT - 1) / MG_CT), nct2 = static_cast<int>((a.H + MG_CT - 1) / MG_CT);
+  // the workspace's lists have room for two offset arrays of kMoeGroupMaxExperts: past
+  // two thirds of that many experts both GEMMs share one
+  const bool two = 3 * (a.E + 1) <= 2 * (kMoeGroupMaxExperts + 1);
+  const int rt1 = mg_tile_rows(a, nct1), rt2 = two ? mg_tile_rows(a, nct2 * a.ks) : rt1;
   MgLists g;
   int32_t* base = reinterpret_cast<int32_t*>(a.cnt);
   g.off = base;
   g.toff = g.off + (a.E + 1);
-  g.list = g.toff + (a.E + 1);
+  g.toff2 = two ? g.toff + (a.E + 1) : g.toff;
+  g.list = g.toff2 + (a.E + 1);
   g.hmax = reinterpret_cast<uint32_t*>(g.list + a.T * a.k);
   g.ex = reinterpret_cast<int32_t*>(g.hmax + a.T * a.k);
   const int T = static_cast<int>(a.T), npairs = static_cast<int>(a.T * a.k), E = static_cast<int>(a.E);
@@ -684,21 +722,20 @@ hipError_t launch_grouped(const MoeArgs& a0, hipStream_t st) {
   const int H = static_cast<int>(a.H);
   auto prep = H <= 2048 ? k_moe_prep<1> : H <= 4096 ? k_moe_prep<2> : H <= 8192 ? k_moe_prep<4> : k_moe_prep<0>;
   hipLaunchKernelGGL(prep, dim3(static_cast<uint32_t>(T)), dim3(256), 0, st, a.router, a.x, a.sel, a.wts, E, a.k, H, g.ex, xs);
-  hipLaunchKernelGGL(k_moe_group, dim3(1), dim3(MG_T), 0, st, a.sel, npairs, E, g);
+  hipLaunchKernelGGL(k_moe_group, dim3(1), dim3(MG_T), 0, st, a.sel, npairs, E, rt1, rt2, g);
   if (hipError_t e = hipGetLastError(); e != hipSuccess) return e;
   // row tiles: at most one partial tile per expert beyond the full ones
-  const int64_t rtmax = (a.T * a.k + MG_RT - 1) / MG_RT + a.E;
-  const int nct1 = static_cast<int>((a.F1 + MG_CT - 1) / MG_CT), nct2 = static_cast<int>((a.H + MG_CT - 1) / MG_CT);
-  if (rtmax * nct1 > 0x7FFFFFFF || rtmax * nct2 * a.ks > 0x7FFFFFFF) return hipErrorInvalidValue;
-  const hipError_t e1 = a.act == XRMM_ACT_SWIGLU_CODE ? mg_launch_s<MG_FC1_SWIGLU>(a, g, nct1, rtmax * nct1, st)
-                                                      : mg_launch_s<MG_FC1_RELU>(a, g, nct1, rtmax * nct1, st);
+  const int64_t rtmax1 = (a.T * a.k + rt1 - 1) / rt1 + a.E, rtmax2 = (a.T * a.k + rt2 - 1) / rt2 + a.E;
+  if (rtmax1 * nct1 > 0x7FFFFFFF || rtmax2 * nct2 * a.ks > 0x7FFFFFFF) return hipErrorInvalidValue;
+  const hipError_t e1 = a.act == XRMM_ACT_SWIGLU_CODE ? mg_launch_s<MG_FC1_SWIGLU>(a, g, rt1, nct1, rtmax1 * nct1, st)
+                                                      : mg_launch_s<MG_FC1_RELU>(a, g, rt1, nct1, rtmax1 * nct1, st);
   if (e1 != hipSuccess) return e1;
   const int64_t hg = a.T * a.k * (a.I / 8);
   if ((hg + 255) / 256 > 0x7FFFFFFF) return hipErrorInvalidValue;
   hipLaunchKernelGGL(k_moe_hsplit, dim3(static_cast<uint32_t>((hg + 255) / 256)), dim3(256), 0, st, a.h, g.hmax, hg,
                      static_cast<int>(a.I / 8));
   if (hipError_t e = hipGetLastError(); e != hipSuccess) return e;
-  if (hipError_t e = mg_launch_s<MG_FC2>(a, g, nct2, rtmax * nct2 * a.ks, st); e != hipSuccess) return e;
+  if (hipError_t e = mg_launch_s<MG_FC2>(a, g, rt2, nct2, rtmax2 * nct2 * a.ks, st); e != hipSuccess) return e;
   hipLaunchKernelGGL(k_moe_combine, dim3(static_cast<uint32_t>((a.T * (a.H / 4) + 255) / 256)), dim3(256), 0, st, a);
   return hipGetLastError();
 }

@@ -1,13 +1,13 @@
 // Grouped-expert QMoE for many tokens (included by xrmm_moe.hip): instead of
 // one pass over an expert's rows per (token, slot) pair, the pairs routed to
 // each expert are gathered into the rows of one GEMM per expert, so every
-// expert matrix is read once per 128 pairs.
+// expert matrix is read once per 128 (or 64) pairs.
 //
 // Launches:
 //  1. k_moe_prep: per token the routing, the row exponent of x, and x split into
 //     its binary16 terms (into yp, which nothing uses before FC2);
-//  2. k_moe_group: per-expert pair counts, offsets, row-tile offsets and the
-//     pair lists (one workgroup; the order of pairs inside a list does not
+//  2. k_moe_group: per-expert pair counts, offsets, the two GEMMs' row-tile offsets and
+//     the pair lists (one workgroup; the order of pairs inside a list does not
 //     change any result, every GEMM row being independent);
 //  3. k_moe_ggemm FC1: rows = an expert's pairs (their tokens' x), columns =
 //     its FC1 rows, K = H; the epilogue applies the row scale, the activation
@@ -35,46 +35,56 @@
 // (split in the tiles, every column tile of an expert split the same rows again:
 // 40 of 180 VALU instructions a step).
 //
-// Tiles. 128 pairs x 256 columns, 8 waves of 2 x 4: a wave owns every other
-// 32-pair MFMA tile (two at most) and 64 columns, so a dequantised weight fragment
-// feeds two MFMA row tiles and experts with 1 .. 128 pairs cost ceil(pairs / 32)
-// MFMA tiles (the 64-pair tiles with two row groups of waves it replaces dequantised
-// every fragment twice and computed their empty rows). Mixtral's experts (H =
-// 4096, I = 14336, 8 experts, 2 taken, blocks of 64), 300 tokens:
-// 1.07 -> 0.74 ms (FC1 750 -> 500 us at best, FC2 338 -> 227, x's exponents by one wave a
-// token 28 us -> part of k_moe_prep's 8.5, combine 12.7 -> 6.5); 16 tokens 630 -> 376 us,
-// 2048 tokens 4.9 -> 3.5 ms. A step's time by wave: 1.7 - 2.0 k cycles of MFMAs and
-// dequantisation, 0.4 k issuing loads, 0.3 k staging, the rest barrier: the two waves of
-// a SIMD overlap only in part. One workgroup per CU leaves a tail where the tiles just
-// pass a round: row scales, ReLU, 250 pairs an expert and 4096 rows (1000 x 2048 x 4096,
-// 8 experts, 2 taken) take 286 us against 255 with 64-pair tiles, two workgroups per CU.
+// Tiles. 128 or 64 pairs x 256 columns, 8 waves of 2 x 4: a wave owns every other
+// 32-pair MFMA tile (two or one) and 64 columns. At 128 pairs a dequantised weight
+// fragment feeds two MFMA row tiles, and experts with 1 .. 128 pairs cost ceil(pairs /
+// 32) MFMA tiles; a workgroup fills a CU (156 KB of LDS, 240 registers). At 64 pairs each
+// weight is dequantised by two waves and staged by 64 bytes a column, but two
+// workgroups share a CU (78 KB, 128 registers), and tiles that would leave CUs idle
+// are twice as many. mg_tile_rows chooses for each of the two GEMMs.
+//
+// Measured (one MI355X; us with the 64-pair tiles that split float32 rows in the tile ->
+// 128-pair tiles only -> both): Mixtral's experts (H = 4096, I = 14336, 8 experts, 2
+// taken, blocks of 64) 16 tokens 621 -> 378 -> 324, 300 tokens 1036 -> 687 -> 686, 2048
+// tokens 4760 -> 3344 -> 3356; row scales, ReLU, 8 experts: 1000 x 2048 x 4096, 2 taken,
+// 239 -> 271 -> 233; 512 x 1024 x 4096, 4 taken, 150 -> 191 -> 161 (the passes that
+// split x and h, 17 us, are not repaid by four FC2 column tiles); 200 x 1024 x 4096, 4
+// taken, 96 -> 128 -> 94. Over 785 sizes 1.36 times as fast as the first, 13 of them 1.5
+// to 8 % slower (55, up to 38 %, with 128-pair tiles alone). A step's time by wave (128 pairs): 1.7 - 2.0 k cycles of MFMAs
+// and dequantisation, 0.4 k issuing loads, 0.3 k staging, the rest barrier: the two waves
+// of a SIMD overlap only in part.
 #pragma once
 
 namespace xrmm {
 namespace {
 
-constexpr int MG_RT = 128;  // pairs per row tile
 constexpr int MG_CT = 256;  // columns per tile
 constexpr int MG_K = 64;    // K step
 constexpr int MG_LD = MG_K + 8;
 constexpr int MG_T = 512;   // threads: 8 waves, 2 (row tiles) x 4 (columns of 64)
-// Weights are staged for several K steps at once, a super-step: 128 bytes of every
-// column (256 codes of 4 bits, 128 of 8).
-template <int BITS>
+// Weights are staged for several K steps at once, a super-step: RT bytes of every
+// column (128: 256 codes of 4 bits, 128 of 8).
+template <int BITS, int RT>
 constexpr int mg_ss() {
-  return BITS == 4 ? 4 : 2;
+  return (BITS == 4 ? 4 : 2) * RT / 128;
 }
-constexpr int MG_ASTAGE = 2 * MG_RT * MG_LD;  // halfs per A stage: hi, then lo (rows of MG_LD)
-constexpr int MG_WSTAGE = MG_CT * 128;        // bytes of a super-step's codes
+template <int RT>
+constexpr int mg_astage() {  // halfs per A stage: hi, then lo (rows of MG_LD)
+  return 2 * RT * MG_LD;
+}
+template <int RT>
+constexpr int mg_wstage() {  // bytes of a super-step's codes
+  return MG_CT * RT;
+}
 // scales of a column and super-step (block mode BKM: 2, 4, 8 = blocks of 32, 64, 128
 // or more codes; longer blocks repeat one scale)
-template <int BITS, int BKM>
+template <int BITS, int BKM, int RT>
 constexpr int mg_sb() {
-  return BKM == 0 ? 0 : BKM == 2 ? 2 * mg_ss<BITS>() : BKM == 4 ? mg_ss<BITS>() : mg_ss<BITS>() / 2;
+  return BKM == 0 ? 0 : BKM == 2 ? 2 * mg_ss<BITS, RT>() : BKM == 4 ? mg_ss<BITS, RT>() : (mg_ss<BITS, RT>() + 1) / 2;
 }
-template <int BITS, int BKM>
+template <int BITS, int BKM, int RT>
 constexpr size_t mg_lds() {
-  return 2 * (MG_ASTAGE * sizeof(_Float16) + MG_WSTAGE + mg_sb<BITS, BKM>() * MG_CT * sizeof(float));
+  return 2 * (mg_astage<RT>() * sizeof(_Float16) + mg_wstage<RT>() + mg_sb<BITS, BKM, RT>() * MG_CT * sizeof(float));
 }
 
 // Block-scale modes of the GEMM: 0 = one scale per row (applied to the row's
@@ -86,7 +96,8 @@ inline int mg_block_mode(int bs) { return bs == 0 ? 0 : bs == 16 ? 1 : bs == 32 
 // Lists of the grouped path, inside the workspace's counter region.
 struct MgLists {
   int32_t* off;    // [E + 1] first list entry of each expert
-  int32_t* toff;   // [E + 1] first row tile of each expert
+  int32_t* toff;   // [E + 1] first row tile of each expert, FC1
+  int32_t* toff2;  // [E + 1] the same of FC2 (toff where both have one tile height)
   int32_t* list;   // [T k] pair indices grouped by expert
   uint32_t* hmax;  // [T k] bits of the largest finite |h| of each pair
   int32_t* ex;     // [T] row exponent of x
@@ -202,11 +213,12 @@ __global__ __launch_bounds__(256) void k_moe_hsplit(float* __restrict__ h, const
   out[8] = lo;
 }
 
-// Pair counts, offsets and lists; also clears hmax. One workgroup of
-// MG_T threads; E <= kMoeGroupMaxExperts (LDS counters).
-__global__ __launch_bounds__(MG_T) void k_moe_group(const int32_t* __restrict__ sel, int npairs, int E, MgLists g) {
+// Pair counts, offsets, lists and the row tiles of rt (FC1) and rt2 (FC2) pairs; also
+// clears hmax. One workgroup of MG_T threads; E <= kMoeGroupMaxExperts (LDS counters).
+__global__ __launch_bounds__(MG_T) void k_moe_group(const int32_t* __restrict__ sel, int npairs, int E, int rt, int rt2,
+                                                    MgLists g) {
   __shared__ int cnt[kMoeGroupMaxExperts];
-  __shared__ int part[MG_T];
+  __shared__ int part[3][MG_T];
   const int tid = threadIdx.x;
   for (int e = tid; e < E; e += MG_T) cnt[e] = 0;
   __syncthreads();
@@ -219,41 +231,39 @@ __global__ __launch_bounds__(MG_T) void k_moe_group(const int32_t* __restrict__ 
   // exclusive scans of the counts and of the row tiles: each thread sums a
   // run of experts, the runs' totals are scanned in LDS
   const int per = (E + MG_T - 1) / MG_T, e0 = tid * per;
-  int s = 0, st = 0;
+  int s[3] = {0, 0, 0};
   for (int e = e0; e < e0 + per && e < E; ++e) {
-    s += cnt[e];
-    st += (cnt[e] + MG_RT - 1) / MG_RT;
+    s[0] += cnt[e];
+    s[1] += (cnt[e] + rt - 1) / rt;
+    s[2] += (cnt[e] + rt2 - 1) / rt2;
   }
-  part[tid] = s;
+#pragma unroll
+  for (int q = 0; q < 3; ++q) part[q][tid] = s[q];
   __syncthreads();
   for (int d = 1; d < MG_T; d <<= 1) {
-    const int v = tid >= d ? part[tid - d] : 0;
+    int v[3];
+#pragma unroll
+    for (int q = 0; q < 3; ++q) v[q] = tid >= d ? part[q][tid - d] : 0;
     __syncthreads();
-    part[tid] += v;
-    __syncthreads();
-  }
-  const int sbase = part[tid] - s;
-  __syncthreads();
-  part[tid] = st;
-  __syncthreads();
-  for (int d = 1; d < MG_T; d <<= 1) {
-    const int v = tid >= d ? part[tid - d] : 0;
-    __syncthreads();
-    part[tid] += v;
+#pragma unroll
+    for (int q = 0; q < 3; ++q) part[q][tid] += v[q];
     __syncthreads();
   }
-  const int tbase = part[tid] - st;
-  int a = sbase, b = tbase;
+#pragma unroll
+  for (int q = 0; q < 3; ++q) s[q] = part[q][tid] - s[q];
   for (int e = e0; e < e0 + per && e < E; ++e) {
-    g.off[e] = a;
-    g.toff[e] = b;
+    g.off[e] = s[0];
+    g.toff[e] = s[1];
+    g.toff2[e] = s[2];
     const int c = cnt[e];
-    a += c;
-    b += (c + MG_RT - 1) / MG_RT;
+    s[0] += c;
+    s[1] += (c + rt - 1) / rt;
+    s[2] += (c + rt2 - 1) / rt2;
   }
-  if (tid == MG_T - 1) {
-    g.off[E] = a;  // the last thread's run ends at E
-    g.toff[E] = b;
+  if (tid == MG_T - 1) {  // the last thread's run ends at E
+    g.off[E] = s[0];
+    g.toff[E] = s[1];
+    g.toff2[E] = s[2];
   }
   __syncthreads();
   // positions: a cursor per expert (the order inside a list is free)
@@ -274,19 +284,23 @@ __device__ __forceinline__ float mg_ror(float v) {
   return __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, v), 0x120 + N, 0xF, 0xF, true));
 }
 
-// One 128-pair x 256-column tile of an expert's matrix; BITS-bit codes, block
+// One tile of RT pairs x 256 columns of an expert's matrix; BITS-bit codes, block
 // mode BKM (mg_block_mode).
-template <int ST, int BITS, int BKM>
-__global__ __launch_bounds__(MG_T, 2) void k_moe_ggemm(MoeArgs a, MgLists g, int nct) {
+template <int ST, int BITS, int BKM, int RT>
+__global__ __launch_bounds__(MG_T, RT == 64 ? 4 : 2) void k_moe_ggemm(MoeArgs a, MgLists g, int nct) {
   constexpr bool FC2 = ST == MG_FC2;
-  constexpr int SS = mg_ss<BITS>(), SB = mg_sb<BITS, BKM>();
+  constexpr int SS = mg_ss<BITS, RT>(), SB = mg_sb<BITS, BKM, RT>();
+  constexpr int MG_ASTAGE = mg_astage<RT>(), MG_WSTAGE = mg_wstage<RT>();
+  constexpr int NI = RT / 64;   // MFMA row tiles of a wave
+  constexpr int CH = RT / 16;   // 16-byte chunks of a column's super-step
+  constexpr int ROT = 64 / CH;  // places a chunk's columns are rotated by, times the chunk
   constexpr int BW = BITS / 4;  // dwords per fragment
   extern __shared__ __align__(16) unsigned char smem[];
   f16* lds = reinterpret_cast<f16*>(smem);                                   // [2] A stages
   uint32_t* wlds = reinterpret_cast<uint32_t*>(lds + 2 * MG_ASTAGE);         // [2] super-steps' codes
   float* slds = reinterpret_cast<float*>(wlds + 2 * (MG_WSTAGE / 4));        // [2][SB][column] scales
-  __shared__ int s_pair[MG_RT];
-  __shared__ float s_ru[MG_RT];  // 2^e per row (epilogue)
+  __shared__ int s_pair[RT];
+  __shared__ float s_ru[RT];  // 2^e per row (epilogue)
   constexpr uint32_t OOB = 0x80000000u;
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -296,25 +310,26 @@ __global__ __launch_bounds__(MG_T, 2) void k_moe_ggemm(MoeArgs a, MgLists g, int
   const int ks2 = FC2 ? a.ks : 1;
   const int sp = static_cast<int>(blockIdx.x) % ks2, tb = static_cast<int>(blockIdx.x) / ks2;
   const int rt = tb / nct, ct = tb % nct;
-  const int total = g.toff[E];
+  const int32_t* toff = FC2 ? g.toff2 : g.toff;
+  const int total = toff[E];
   if (rt >= total) return;  // uniform: the grid is an upper bound of the row tiles
   // expert of this row tile: the last e with toff[e] <= rt
   int lo = 0, hi = E - 1;
   while (lo < hi) {
     const int mid = (lo + hi + 1) >> 1;
-    if (g.toff[mid] <= rt) lo = mid;
+    if (toff[mid] <= rt) lo = mid;
     else hi = mid - 1;
   }
   const int e = lo;
   // the expert's pairs over its row tiles in equal whole 32s (260 pairs: 96, 96, 68)
-  const int npe = g.off[e + 1] - g.off[e], nte = g.toff[e + 1] - g.toff[e];
+  const int npe = g.off[e + 1] - g.off[e], nte = toff[e + 1] - toff[e];
   const int rpt = ((npe + nte - 1) / nte + 31) & ~31;
-  const int lb = g.off[e] + (rt - g.toff[e]) * rpt;  // first list entry of the tile
+  const int lb = g.off[e] + (rt - toff[e]) * rpt;  // first list entry of the tile
   const int nrow = min(rpt, g.off[e + 1] - lb);
   const int Kd = static_cast<int>(FC2 ? a.I : a.H);   // reduction length
   const int Nd = static_cast<int>(FC2 ? a.H : a.F1);  // rows of the expert matrix
   const int n0 = ct * MG_CT;
-  if (tid < MG_RT) {
+  if (tid < RT) {
     const int p = tid < nrow ? g.list[lb + tid] : -1;
     s_pair[tid] = p;
     int ex = 0;
@@ -351,13 +366,13 @@ __global__ __launch_bounds__(MG_T, 2) void k_moe_ggemm(MoeArgs a, MgLists g, int
   //    scales of column t.
   const int st_t = tid & 255;
   struct ARegs {
-    u32x4 v[4][2];
+    u32x4 v[2 * NI][2];
   };
-  const float* Arow[4];
+  const float* Arow[2 * NI];
   {
     const float* Asrc = FC2 ? a.h : a.yp;  // FC1: x's terms
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
+    for (int i = 0; i < 2 * NI; ++i) {
       const int r = (st_t >> 3) + 32 * i, p = s_pair[r] < 0 ? s_pair[0] : s_pair[r];
       Arow[i] = Asrc + (FC2 ? static_cast<int64_t>(p) * a.I : static_cast<int64_t>(p / a.k) * a.H) + (st_t & 7) * 4;
     }
@@ -366,7 +381,7 @@ __global__ __launch_bounds__(MG_T, 2) void k_moe_ggemm(MoeArgs a, MgLists g, int
   const int nsub = (nrow + 31) / 32;
   auto aload = [&](ARegs& r, int ks) {
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
+    for (int i = 0; i < 2 * NI; ++i) {
       if (i >= nsub) break;
       const float* pa = Arow[i] + (kstep0 + ks) * MG_K;
       r.v[i][0] = *reinterpret_cast<const u32x4*>(pa);
@@ -376,10 +391,10 @@ __global__ __launch_bounds__(MG_T, 2) void k_moe_ggemm(MoeArgs a, MgLists g, int
   auto astore = [&](const ARegs& r, int stage) {
     f16* Ah = lds + stage * MG_ASTAGE + (st_t >> 3) * MG_LD + (st_t & 7) * 8;
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
+    for (int i = 0; i < 2 * NI; ++i) {
       if (i >= nsub) break;
       *reinterpret_cast<u32x4*>(Ah + 32 * i * MG_LD) = r.v[i][0];
-      *reinterpret_cast<u32x4*>(Ah + (MG_RT + 32 * i) * MG_LD) = r.v[i][1];
+      *reinterpret_cast<u32x4*>(Ah + (RT + 32 * i) * MG_LD) = r.v[i][1];
     }
   };
   // scales: [E, Nd] (row scales) or [E, Nd, Kd / block_size]
@@ -387,17 +402,17 @@ __global__ __launch_bounds__(MG_T, 2) void k_moe_ggemm(MoeArgs a, MgLists g, int
   const float* S = FC2 ? a.s2 + static_cast<int64_t>(e) * a.H * nblk : a.s1 + static_cast<int64_t>(e) * a.F1 * nblk;
   const rsrc_t rS = mk_rsrc(S, static_cast<uint32_t>(Nd) * static_cast<uint32_t>(nblk) * 4u);
   struct WRegs {
-    u32x4 v[8];
+    u32x4 v[CH];
     uint32_t s[SB ? SB : 1];
   };
-  // codes i0 .. i1 - 1 (of a thread's eight) of super-step u, with the first its scales;
+  // chunks i0 .. i1 - 1 (of a thread's CH) of super-step u, with the first its scales;
   // past the row: zeros
   auto wload = [&](WRegs& r, int u, int i0, int i1) __attribute__((always_inline)) {
-    const uint32_t o = static_cast<uint32_t>((kstep0 + u * SS) * MG_K * BITS / 8 + (st_t & 7) * 16);
+    const uint32_t o = static_cast<uint32_t>((kstep0 + u * SS) * MG_K * BITS / 8 + (st_t & (CH - 1)) * 16);
     const uint32_t past = u * SS < ksteps && o < rowb ? 0u : OOB;
 #pragma unroll
     for (int i = i0; i < i1; ++i) {
-      const int c = n0 + (st_t >> 3) + 32 * i;
+      const int c = n0 + st_t / CH + 256 / CH * i;
       r.v[i] = bld16(rB, ((c < Nd ? static_cast<uint32_t>(c) * rowb : OOB) | past) + o, 0);
     }
     if (i0 > 0) return;
@@ -425,10 +440,10 @@ __global__ __launch_bounds__(MG_T, 2) void k_moe_ggemm(MoeArgs a, MgLists g, int
   // writes at once fall in different banks
   auto wstore = [&](const WRegs& r, int buf) {
     uint32_t* W = wlds + buf * (MG_WSTAGE / 4);
-    const int c = st_t & 7;
+    const int c = st_t & (CH - 1);
 #pragma unroll
-    for (int i = 0; i < 8; ++i) {
-      const int col = ((st_t >> 3) + 32 * i + 8 * c) & (MG_CT - 1);
+    for (int i = 0; i < CH; ++i) {
+      const int col = (st_t / CH + 256 / CH * i + ROT * c) & (MG_CT - 1);
       const u32x4 v = r.v[i];
       if constexpr (BW == 1) {
         uint32_t* d = W + 4 * c * MG_CT + col;
@@ -473,10 +488,10 @@ __global__ __launch_bounds__(MG_T, 2) void k_moe_ggemm(MoeArgs a, MgLists g, int
 
   // block sums (acc) and, with block scales, the scaled running sums (yacc), of
   // the wave's row tiles wm, wm + 2
-  f32x16 acc[2][2];
-  float yacc[BKM ? 2 : 1][BKM ? 2 : 1][16];
+  f32x16 acc[NI][2];
+  float yacc[BKM ? NI : 1][BKM ? 2 : 1][16];
 #pragma unroll
-  for (int i = 0; i < 2; ++i)
+  for (int i = 0; i < NI; ++i)
 #pragma unroll
     for (int j = 0; j < 2; ++j)
 #pragma unroll
@@ -507,13 +522,13 @@ __global__ __launch_bounds__(MG_T, 2) void k_moe_ggemm(MoeArgs a, MgLists g, int
   // step t of its super-step, on A stage `stage` and weight buffer `buf`
   auto mfmas = [&](auto na, int stage, int buf, int t) __attribute__((always_inline)) {
     const f16* Ah = lds + stage * MG_ASTAGE;
-    const f16* Al = Ah + MG_RT * MG_LD;
+    const f16* Al = Ah + RT * MG_LD;
     const uint32_t* W = wlds + buf * (MG_WSTAGE / 4) + 8 * t * MG_CT * BW;
     const float* sc = slds + buf * SB * MG_CT + lcol;
 #pragma unroll
     for (int kk = 0; kk < MG_K / 16; ++kk) {
       const int ko = kk * 16 + (lane >> 5) * 8;
-      f16x8 fh[2], fl[2];
+      f16x8 fh[NI], fl[NI];
 #pragma unroll
       for (int i = 0; i < na; ++i) {
         const int ar = (wm + 2 * i) * 32 + (lane & 31);
@@ -525,7 +540,7 @@ __global__ __launch_bounds__(MG_T, 2) void k_moe_ggemm(MoeArgs a, MgLists g, int
 #pragma unroll
       for (int j = 0; j < 2; ++j) {
         // codes k = ko .. ko + 7 of column lcol + 32 j: fragment ko / 8
-        const f16x8 fb = dq(W + ((ko >> 3) * MG_CT + ((lcol + 32 * j + 8 * chunk) & (MG_CT - 1))) * BW);
+        const f16x8 fb = dq(W + ((ko >> 3) * MG_CT + ((lcol + 32 * j + ROT * chunk) & (MG_CT - 1))) * BW);
 #pragma unroll
         for (int i = 0; i < na; ++i) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(fh[i], fb, first ? zero16 : acc[i][j], 0, 0, 0);
 #pragma unroll
@@ -543,10 +558,12 @@ __global__ __launch_bounds__(MG_T, 2) void k_moe_ggemm(MoeArgs a, MgLists g, int
   // Order of the K steps: column tile ct starts at super-step ct of its range and wraps
   // around. The tiles run side by side; all at the same k, they would read the same
   // 128 bytes of every row, whose stride of H / 2 bytes lands on few memory channels
-  // (1.6 TB/s). The start is a whole number of scale blocks.
+  // (1.6 TB/s). The start is a whole number of scale blocks. Not so for 64-pair tiles of
+  // experts with many pairs: the L2 then serves a row's activations to all column tiles
+  // at once (block scales, 60 pairs an expert and more: 5 % faster without, up to 12).
   const int ru = BKM == 8 && bsteps > SS ? bsteps : SS;
   const int nru = ksteps / ru;
-  const int first_step = nru > 1 ? ct % nru * ru : 0;
+  const int first_step = nru > 1 && !(RT == 64 && npe > 16) ? ct % nru * ru : 0;
   // role 0 (waves 0 .. 3): weights; 1: activations. na: the wave's row tiles that hold
   // pairs, 2, 1 or none (it then only stages). All loops have the same barriers.
   auto loop = [&](auto role, auto na) __attribute__((always_inline)) {
@@ -554,7 +571,7 @@ __global__ __launch_bounds__(MG_T, 2) void k_moe_ggemm(MoeArgs a, MgLists g, int
     WRegs wr;
     int p = first_step, buf = 0;  // the step, its weight buffer
     if constexpr (role == 0) {
-      wload(wr, p / SS, 0, 8);
+      wload(wr, p / SS, 0, CH);
       wstore(wr, 0);
     } else {
       aload(ar, p);
@@ -568,12 +585,12 @@ __global__ __launch_bounds__(MG_T, 2) void k_moe_ggemm(MoeArgs a, MgLists g, int
         // the super-step after this one (the row's first after its last), over its first
         // three steps (all eight at once hold up the activations' loads: 1.5 k cycles)
         const int u = (p / SS + 1) * SS < ksteps ? p / SS + 1 : 0;
-        if constexpr (SS == 4) {
+        if constexpr (SS == 4 && CH == 8) {
           if (t == 0) wload(wr, u, 0, 3);
           if (t == 1 || (last && t < 1)) wload(wr, u, 3, 6);  // the row may end inside the super-step
           if (t == 2 || (last && t < 2)) wload(wr, u, 6, 8);
         } else {
-          if (t == 0) wload(wr, u, 0, 8);
+          if (t == 0) wload(wr, u, 0, CH);
         }
       } else {
         aload(ar, next);
@@ -603,12 +620,11 @@ __global__ __launch_bounds__(MG_T, 2) void k_moe_ggemm(MoeArgs a, MgLists g, int
     const int na = ((nrow + 31) / 32 - wm + 1) / 2;
     using I0 = std::integral_constant<int, 0>;
     using I1 = std::integral_constant<int, 1>;
-    using I2 = std::integral_constant<int, 2>;
     if (wm == 0) {
-      if (na >= 2) loop(I0{}, I2{});
+      if (NI == 2 && na >= 2) loop(I0{}, std::integral_constant<int, NI>{});
       else loop(I0{}, I1{});  // a tile holds a pair
     } else {
-      if (na >= 2) loop(I1{}, I2{});
+      if (NI == 2 && na >= 2) loop(I1{}, std::integral_constant<int, NI>{});
       else if (na == 1) loop(I1{}, I1{});
       else loop(I1{}, I0{});
     }
@@ -616,7 +632,7 @@ __global__ __launch_bounds__(MG_T, 2) void k_moe_ggemm(MoeArgs a, MgLists g, int
 
   // ---- epilogue: lane holds D[8 (q / 4) + 4 (lane / 32) + q % 4][lane % 32]
 #pragma unroll
-  for (int i = 0; i < 2; ++i) {
+  for (int i = 0; i < NI; ++i) {
     if (wm + 2 * i >= nsub) break;  // no pair in the row tile
     const int r0 = (wm + 2 * i) * 32 + 4 * (lane >> 5);
     auto value = [&](int j, int q, float sc) {
