@@ -197,8 +197,8 @@ __global__ __launch_bounds__(256) void k_moe_prep(const float* __restrict__ rout
 
 // h [T k][I] into its terms in place, eight values per thread; the row exponent from
 // the pair's largest |h| (FC1's atomic maximum). The eight threads that exchange
-// places inside 256 bytes are lanes of one wave (I % 64 == 0), whose load
-// instructions have all returned before its first store is issued.
+// places inside 256 bytes are lanes of one wave (I % 64 == 0): the fence and the wave
+// barrier keep every lane's loads before the first lane's store.
 __global__ __launch_bounds__(256) void k_moe_hsplit(float* __restrict__ h, const uint32_t* __restrict__ hmax, int64_t groups,
                                                     int gpr) {
   const int64_t g = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x;
@@ -208,6 +208,8 @@ __global__ __launch_bounds__(256) void k_moe_hsplit(float* __restrict__ h, const
   f16x8 hi, lo;
   mg_load8(h + g * 8, x);
   mg_terms(x, scale, hi, lo);
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  __builtin_amdgcn_wave_barrier();
   f16x8* out = reinterpret_cast<f16x8*>(h + (g >> 3) * 64) + (g & 7);
   out[0] = hi;
   out[8] = lo;
