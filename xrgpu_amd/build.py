@@ -88,11 +88,21 @@ def _run(cmd, verbose):
 
 
 def build_front(cxx, verbose):
-    """The torch extension: host code against the installed torch's headers."""
-    import torch
+    """The torch extension: host code against the installed torch's headers. Left out,
+    with a note, where torch, its headers or Python's are not installed (the C library
+    and the runner need none of them; ops.py then makes every call itself)."""
+    try:
+        import torch
+    except ImportError:
+        print("xrgpu_amd: no torch here, the native front end of ops.py is not built", file=sys.stderr)
+        return
     t = os.path.dirname(torch.__file__)
     inc = [os.path.join(t, "include"), os.path.join(t, "include", "torch", "csrc", "api", "include"),
            sysconfig.get_paths()["include"]]
+    for path in (os.path.join(inc[0], "ATen", "ATen.h"), os.path.join(inc[2], "Python.h")):
+        if not os.path.exists(path):
+            print(f"xrgpu_amd: no {path}, the native front end of ops.py is not built", file=sys.stderr)
+            return
     _run([cxx, "-O2", "-std=c++17", "-fPIC", "-shared", "-Wall", "-Wno-maybe-uninitialized",
           f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}", *[a for i in inc for a in ("-I", i)],
           os.path.join(CSRC, "xrmm_torch.cpp"), "-o", FRONT + ".tmp", "-L", os.path.join(t, "lib"), "-ltorch_python",
