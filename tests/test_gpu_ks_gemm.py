@@ -77,6 +77,40 @@ def test_bnb4_nonfinite(gpu, qt):
     assert np.allclose(got[fin].astype(np.float64), ref[fin].astype(np.float64), rtol=2e-3, atol=1e-3)
 
 
+@pytest.mark.parametrize("qt", [1, 0])
+def test_bnb4_codebook_precision(gpu, qt):
+    """Two products that nearly cancel show the codebook's own error: the weights are
+    held to a quarter of float32's 2^-24 (a float32 table rounds to half of it), whose
+    share in the difference is at most 0.5 units of 2^-24 of the magnitudes, beside the
+    roundings of the scale and of the result."""
+    book = (Q.NF4 if qt == 1 else Q.FP4).astype(np.float64)
+    rows = []
+    for c1 in range(16):
+        for c2 in range(16):
+            a1 = np.arange(1025, 2049, dtype=np.float64)
+            if c1 == c2 or book[c1] == 0 or book[c2] == 0:
+                continue
+            a2 = -np.round(a1 * book[c1] / book[c2])
+            ok = np.abs(a2) <= 2048  # exact in binary16
+            if ok.any():
+                i = np.abs(a1 * book[c1] + a2 * book[c2])[ok].argmin()
+                rows.append((c1, c2, a1[ok][i], a2[ok][i]))
+    M, K, bs = len(rows), 32, 32
+    zero = 7 if qt == 1 else 0
+    a, codes = np.zeros((M, K)), np.full((M, K), zero)
+    for m, (c1, c2, a1, a2) in enumerate(rows):
+        a[m, :2], codes[m, :2] = (a1, a2), (c1, c2)
+    b = (codes[:, 0::2] << 4 | codes[:, 1::2]).astype(np.uint8)
+    s = np.random.default_rng(qt).uniform(0.3, 1.7, M).astype(np.float16)
+    assert ops().bnb4_kernel(M, K, M, bs, qt, 1, torch.float16) == "bnb4_gemm"
+    got = np.diag(ops().matmul_bnb4(dev(a.astype(np.float16)), dev(b.reshape(-1)), dev(s), K=K, N=M, block_size=bs,
+                                    quant_type=qt).cpu().numpy()).astype(np.float64)
+    terms = a[:, :2] * book[codes[:, :2]] * s.astype(np.float64)[:, None]
+    exact, mag = terms.sum(1), np.abs(terms).sum(1)
+    lim = np.abs(exact) * (2.0 ** -11 + 2.0 ** -22) + mag * 0.5 * 2.0 ** -24 + 2.0 ** -25
+    assert np.all(np.abs(got - exact) <= lim), float(((np.abs(got - exact) - np.abs(exact) * 2.0 ** -11) / mag).max() * 2 ** 24)
+
+
 I8A = [  # M, K, N, block, zero points, bias, dtype
     (2049, 128, 1030, 32, True, True, np.float16),   # one pair of steps
     (33, 1024, 8200, 64, True, False, np.float32),

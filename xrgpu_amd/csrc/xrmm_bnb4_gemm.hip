@@ -11,15 +11,26 @@ namespace {
 
 struct Planes {
   uint32_t t[16];
+  float unscale;
 };
 
-// The codebook, times 2^15, as two binary16 terms of each value's own sign:
+// Factors of the codebooks. Two binary16 terms of one sign hold 22 bits of a value:
+// at 2^15 the float32 codebooks' values were up to 1.6 units of 2^-24 off. A factor
+// that is not a power of two moves all of them; of 32 million float32 factors in 2^14 ..
+// 2^15 these leave 0.28 units at most for NF4, none for FP4 (nearly 192 times a power
+// of two, FP4's common denominator), with every lo at least 2^-13 (a normal binary16
+// value). What the factor's inverse and its product with a block's scale round is common
+// to a block's weights.
+constexpr double kNF4Factor = 0x1.8d1becp+14, kFP4Factor = 0x1.f80018p+14;
+
+// The codebook, times the factor, as two binary16 terms of each value's own sign:
 // hi the largest magnitude below the value, lo the rest (rounded to nearest,
 // never zero unless the value is), split into their low and high bytes.
-Planes planes(const float (&book)[16]) {
+Planes planes(const float (&book)[16], double factor) {
   Planes p{};
+  p.unscale = static_cast<float>(1.0 / factor);
   for (int c = 0; c < 16; ++c) {
-    const double v = std::fabs(static_cast<double>(book[c])) * 32768.0;
+    const double v = std::fabs(static_cast<double>(book[c])) * factor;
     double hi = 0.0;
     if (v > 0.0) {
       int e = 0;
@@ -53,7 +64,7 @@ bool bnb4_gemm_ok(const Bnb4Args& a) {
 }
 
 hipError_t launch_bnb4_gemm(const Bnb4Args& a, const float (&nf4)[16], const float (&fp4)[16], hipStream_t st) {
-  static const Planes nf = planes(nf4), fp = planes(fp4);
+  static const Planes nf = planes(nf4, kNF4Factor), fp = planes(fp4, kFP4Factor);
   ks::Args g{};
   g.A = a.A;
   g.B = a.B;
@@ -67,6 +78,7 @@ hipError_t launch_bnb4_gemm(const Bnb4Args& a, const float (&nf4)[16], const flo
   g.kb = static_cast<int>(a.K / a.bs);
   const Planes& p = a.qt == 1 ? nf : fp;
   for (int i = 0; i < 16; ++i) g.tbl[i] = p.t[i];
+  g.unscale = p.unscale;
   const int cus = device_cus();
   const ks::Plan pl = ks::plan(a.M, a.N, a.K, cus > 0 ? cus : 256, 4);
   g.nrt = pl.nrt;

@@ -8,8 +8,8 @@
 //    the sum of two binary16 terms of its own sign (hi rounded towards zero and
 //    below the value, lo the rest), so +-Inf activations meet no zero term that
 //    the float32 product would not have; both terms go through the matrix cores.
-//    Values are scaled by 2^15 (undone in the block scale), which keeps lo out
-//    of binary16's subnormal range.
+//    Values are scaled (undone in the block scale) by a factor near 2^15, chosen
+//    for each codebook so that the two terms hold its values to 0.3 of 2^-24.
 //  * int8-activation MatMulNBits (KS_Q8): activation codes and code - zero
 //    point are exact binary16 integers, so a block's sum is the exact integer
 //    the int8 dot product gives (below 2^24); the block sums, times their weight
@@ -56,6 +56,7 @@ struct Args {
   const uint8_t* Z;   // KS_Q8: packed zero points [N][zrow], or null (8)
   const void* bias;   // [N] or null
   void* Y;            // [M][N]
+  float unscale;      // KS_BNB: one over the codebook's factor
   uint32_t tbl[16];   // KS_BNB: the codebook as four byte planes of 16: hi low, hi high, lo low, lo high byte
   int M, K, N, kb, bs, lbs, zrow, nrt;  // bs = 2^lbs
 };
@@ -235,7 +236,7 @@ __global__ __launch_bounds__(THREADS, 2) void k_gemm_ks(Args a) {
     if constexpr (sizeof(T) == 4) v = __builtin_bit_cast(float, r.s[i]);
     else if constexpr (VEC && SN > 1) v = static_cast<float>(__builtin_bit_cast(f16, static_cast<uint16_t>(r.s[i >> 1] >> (16 * (i & 1)))));
     else v = static_cast<float>(__builtin_bit_cast(f16, static_cast<uint16_t>(r.s[i])));
-    return Q8 ? v : v * 0x1p-15f;
+    return Q8 ? v : v * a.unscale;
   };
   auto zero_of = [&](const WRegs& r, int s, int t, int f) -> uint32_t {
     if constexpr (!ZP) return 8u;
