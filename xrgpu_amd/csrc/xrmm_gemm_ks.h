@@ -527,7 +527,8 @@ template <typename T, int KIND, int IM, int KG, bool VEC, bool ZP>
 hipError_t launch_bkm(const Args& a, int64_t grid, hipStream_t st) {
   if (a.bs == 32) return launch_one<T, KIND, IM, KG, 2, VEC, ZP>(a, grid, st);
   if (a.bs == 64) return launch_one<T, KIND, IM, KG, 4, VEC, ZP>(a, grid, st);
-  return launch_one<T, KIND, IM, KG, 8, VEC, ZP>(a, grid, st);
+  if constexpr (VEC) return launch_one<T, KIND, IM, KG, 8, VEC, ZP>(a, grid, st);
+  return hipErrorInvalidValue;  // blocks of 128 and more divide K, which is then a multiple of 128
 }
 
 template <typename T, int KIND, int IM, int KG>
