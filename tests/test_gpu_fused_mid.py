@@ -28,8 +28,8 @@ def weights(rng, N, K, bs, zp):
     Z = None
     if zp == "packed":
         Z = rng.integers(0, 256, (N, (kb + 1) // 2), dtype=np.uint8)
-    elif zp == "float":
-        Z = rng.uniform(4, 12, (N, kb)).astype(np.float16)
+    elif zp is not None:
+        Z = rng.uniform(4, 12, (N, kb)).astype(np.float32 if zp == "float32" else np.float16)
     return B, S, Z
 
 
@@ -41,10 +41,42 @@ CASES = [  # M, K, N, Nkv, block, zero points, skip
     (385, 320, 9000, 136, 64, "packed", True),  # past one round of narrow tiles: wide ones
     (257, 96, 11500, 64, 32, "float", False),
 ]
+# past one round of narrow tiles, too few 256 x 256 ones: the wide form
+WIDE_QKV = [(385, 128, 9000, 136, 32, None, False), (300, 320, 12001, 40, 64, "float32", True)]
+WIDE_MLP = [
+    (333, 192, 5632, 0, 32, None, True),
+    (257, 96, 5500, 0, 32, "packed", False),   # a row tile of one row, a column tile not whole
+    (256, 320, 11001, 0, 64, "float", True),   # odd width, five steps
+    (300, 136, 6000, 0, 64, "float32", False),  # a last block that is not whole
+]
 
 
+def form(op, M, N, Nkv):
+    """The tiles the dispatch picks for normalised rows and blocks of 32 and more (the
+    family's name, gemm_q4_fused, also covers the 128 x 128 kernel that has no workspace)."""
+    def up(a, b):
+        return -(-a // b)
 
-@pytest.mark.parametrize("M,K,N,Nkv,bs,zp,skip", CASES)
+    def cols(w):
+        return up(N, w // 2) if op == "mlp" else up(N, w) + 2 * up(Nkv, w)
+    if M >= 128 and up(M, 256) * cols(256) >= 128:
+        return "big"
+    return "narrow" if up(M, 128) * cols(128) <= torch.cuda.get_device_properties(0).multi_processor_count else "wide"
+
+
+def test_forms(gpu):
+    """The cases below reach every form they are meant for."""
+    for op, wide in (("qkv", WIDE_QKV), ("mlp", WIDE_MLP)):
+        assert {form(op, *c[:1], *c[2:4]) for c in wide} == {"wide"}
+        for M, K, N, Nkv, bs, zp, skip in wide:
+            assert ops().fused_workspace_bytes(op, M, K, N, Nkv, block_size=bs, skip=skip) > 0
+            if op == "mlp":  # (the query takes one width, Qkv has two)
+                assert ops().select_kernel("MatMulNBitsMlp", M, K, N, 4, bs) == "gemm_q4_fused"
+    assert {form("qkv", *c[:1], *c[2:4]) for c in CASES} == {"narrow", "wide"}
+    assert {form("mlp", *c[:1], *c[2:4]) for c in CASES} == {"narrow", "big"}
+
+
+@pytest.mark.parametrize("M,K,N,Nkv,bs,zp,skip", CASES + WIDE_QKV)
 def test_qkv(gpu, M, K, N, Nkv, bs, zp, skip):
     rng = np.random.default_rng(M + K + N)
     A = rng.standard_normal((M, K)).astype(np.float16)
@@ -64,7 +96,7 @@ def test_qkv(gpu, M, K, N, Nkv, bs, zp, skip):
     assert np.array_equal(got[3].cpu().numpy(), r)
 
 
-@pytest.mark.parametrize("M,K,N,Nkv,bs,zp,skip", CASES)
+@pytest.mark.parametrize("M,K,N,Nkv,bs,zp,skip", CASES + WIDE_MLP)
 def test_mlp(gpu, M, K, N, Nkv, bs, zp, skip):
     rng = np.random.default_rng(M + K + N + 1)
     A = rng.standard_normal((M, K)).astype(np.float16)
@@ -82,6 +114,26 @@ def test_mlp(gpu, M, K, N, Nkv, bs, zp, skip):
     ref = h[0] / (1 + np.exp(-h[0])) * h[1]
     ok, err, lim = O.tolerance_ok(y.cpu().numpy(), ref.astype(np.float16), np.float16)
     assert ok, (err, lim)
+
+
+@pytest.mark.parametrize("M,N", [(70, 64), (333, 5632)])  # narrow, wide
+def test_unaligned_output(gpu, M, N):
+    """An output two bytes past a 16-byte boundary (the C entry takes any) is written element by element."""
+    from xrgpu_amd import _native as nat
+    K, bs = 128, 32
+    rng = np.random.default_rng(M)
+    A = dev(rng.standard_normal((M, K)).astype(np.float16))
+    g, u = ([dev(t) for t in weights(rng, N, K, bs, None)[:2]] for _ in range(2))
+    gm = dev(rng.uniform(0.5, 1.5, K).astype(np.float16))
+    want, _ = ops().matmul_nbits_mlp(A, *g, *u, norm_scale=gm, block_size=bs)
+    buf = torch.full((M * N + 16,), 7.0, dtype=torch.float16, device="cuda")
+    ws = torch.empty(ops().fused_workspace_bytes("mlp", M, K, N, block_size=bs), dtype=torch.uint8, device="cuda")
+    nat.check(nat.lib().xrmm_matmul_nbits_mlp_ws(
+        A.data_ptr(), None, gm.data_ptr(), g[0].data_ptr(), g[1].data_ptr(), None, None, u[0].data_ptr(), u[1].data_ptr(),
+        None, None, nat.UNSPECIFIED, buf.data_ptr() + 2, None, M, K, N, 4, bs, 1e-5, nat.ACT["silu"], nat.F16, ws.data_ptr(),
+        ws.numel(), torch.cuda.current_stream().cuda_stream))
+    assert torch.equal(buf[1:1 + M * N].view(M, N), want)
+    assert (buf[:1] == 7).all() and (buf[1 + M * N:] == 7).all()
 
 
 def test_two_gib_of_activations(gpu):

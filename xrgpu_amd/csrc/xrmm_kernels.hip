@@ -18,8 +18,15 @@
 //                not fill the chip. LDS-tiled MFMA GEMM with 128 x 128 tiles:
 //                activation tiles and weight tiles dequantised to fp16 are
 //                staged in LDS and fed to v_mfma_f32_32x32x16_f16.
-//  * k_gemm_fused  Qkv / Mlp, 16 < M (xrmm_gemm_fused.h): the same tiling with
-//                the RMS prologue, residual and SwiGLU epilogue fused.
+//  * k_gemm_mid  Qkv / Mlp, 16 < M (Mlp: 64 < M), rows normalised beforehand into a
+//                workspace or nothing to normalise (xrmm_gemm_mid.h): 128-row tiles on
+//                the double-buffered pipeline, while 256 x 256 tiles would not fill the
+//                chip.
+//  * k_gemm_fused  the same calls without that workspace, or with blocks of 16
+//                (xrmm_gemm_fused.h): k_gemm_q4's tiling with the RMS prologue,
+//                residual and SwiGLU epilogue fused.
+//  * k_gemm_thin  17 .. 64 rows (xrmm_gemm_thin.h): weights straight into the MFMA
+//                operands.
 //  * k_gemm_q4_big  M >= 128, fp16, 4-bit (xrmm_gemm.h): 256 x 256 tiles on
 //                eight waves, dequantisation interleaved with the MFMAs.
 //  * k_generic   every other geometry (fp32, 2/8-bit, float zero points with a
@@ -727,7 +734,7 @@ const char* kernel_name(Kernel k) {
     case K_GEMV_F32: return "gemv_q4_f32";
     case K_GEMM_Q4: return "gemm_q4_mfma";
     case K_GEMM_BIG: return "gemm_q4_big";
-    case K_GEMM_FUSED: return "gemm_q4_fused";
+    case K_GEMM_FUSED: return "gemm_q4_fused";  // k_gemm_mid or k_gemm_fused (gemm_mid_ok)
     case K_GEMM_BIG_FUSED: return "gemm_q4_big_fused";
     case K_GEMM_THIN: return "gemm_q4_thin";
     case K_GEMM_F32X: return "gemm_f32_mfma";
