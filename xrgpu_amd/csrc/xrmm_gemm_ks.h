@@ -33,7 +33,8 @@
 // activations, 384 x 4096 x 4096, blocks of 32: 223 -> 40.5 us (the GEMV's lanes
 // read every activation code once per column). What bounds it: VALU issue (codebook
 // decode, scaling of the block sums, staging) and the matrix cores, which two waves
-// per SIMD overlap only in part (VALU 45 %, MFMA 35 % busy in a full round).
+// per SIMD overlap only in part. Counters over the kernel: NF4, 172 workgroups, on
+// their CUs VALU issue 56 % and MFMA 38 % of the cycles; int8, 256 workgroups, 49 and 12 %.
 #pragma once
 
 #include <atomic>
