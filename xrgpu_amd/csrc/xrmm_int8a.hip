@@ -36,11 +36,12 @@ __global__ __launch_bounds__(I8T) void k_i8a_quant(Int8aArgs a) {
   const int64_t m = blk / nb, b = blk % nb;
   const T* src = static_cast<const T*>(a.A) + m * a.K + b * kI8aBlock;
   const float x0 = static_cast<float>(src[2 * lane]), x1 = static_cast<float>(src[2 * lane + 1]);
-  float mx = fmaxf(fabsf(x0), fabsf(x1));
+  // magnitudes order like their bit patterns, NaN above infinity above every finite value
+  auto mag = [](float x) { return __builtin_bit_cast(uint32_t, x) & 0x7FFFFFFFu; };
+  uint32_t mb = max(mag(x0), mag(x1));
 #pragma unroll
-  for (int off = 32; off > 0; off >>= 1) mx = fmaxf(mx, __shfl_xor(mx, off, 64));
-  const bool finite = __builtin_isfinite(x0) && __builtin_isfinite(x1);  // fmaxf passes over NaN
-  const float scale = __builtin_amdgcn_ballot_w64(!finite) != 0 ? __builtin_nanf("") : __fdiv_rn(mx, 127.f);
+  for (int off = 32; off > 0; off >>= 1) mb = max(mb, static_cast<uint32_t>(__shfl_xor(static_cast<int>(mb), off, 64)));
+  const float scale = mb >= 0x7F800000u ? __builtin_nanf("") : __fdiv_rn(__builtin_bit_cast(float, mb), 127.f);
   auto code = [&](float x) -> int8_t {
     if (scale == 0.f) return 0;
     const float q = rintf(__fdiv_rn(x, scale));
