@@ -59,7 +59,7 @@ inline int64_t moe_list_words(int64_t T, int64_t k) { return 2 * (kMoeGroupMaxEx
 // K splits of the grouped path's FC2 GEMM: enough for about 512 tiles of 64 pairs x 256
 // columns (two workgroups per CU; 128-pair tiles, one per CU, are half as many) when the
 // pairs would make fewer, four at most, each split at least 16 steps of 64. From the
-// geometry alone, so the workspace bound and the launch agree. (Two splits fewer save
+// geometry alone, so the workspace bound and the launch agree. (Fewer splits save
 // 11 of 714 us on 300 tokens of Mixtral's experts, but longer float32 sums: 3.4e-7 from
 // the exact result against 3.1e-7.)
 inline int64_t moe_group_fc2_splits(int64_t T, int64_t k, int64_t H, int64_t I) {
